@@ -240,8 +240,9 @@ VXT_API int vxt_hip_dequant_rows_dev(void* ctx, void* tensor, uint32_t row0, uin
  * (vxt_cb4_ffn_gu_nr2_m1, vxt_cb4_fast.metal:212-287) and, for batches, its
  * GEMM + vxt_cb4_swiglu_batch (vxt_cb4_fast_ops.metal:236-262); the CPU
  * step is forward_multi + the activation loop (llm_cpu.rs:448-464).
- * batch_m 1..2 is one fused launch; larger batches stage g and u (f32) in
- * the context workspace, with the workspace rules of vxt_hip_matmul_dev. */
+ * Small batches are one fused launch; the others stage g and u (f32) in the
+ * context workspace.  From batch_m 3 the workspace of the staged form is
+ * reserved either way, with the rules of vxt_hip_matmul_dev. */
 VXT_API int vxt_hip_ffn_glu_dev(void* ctx, void* tensor, const void* x, uint32_t x_dtype, uint32_t batch_m,
                                 void* act, uint32_t act_dtype, uint32_t act_stride, uint32_t activation,
                                 void* stream, char* err, size_t err_cap);
@@ -556,9 +557,10 @@ VXT_API int vxt_hip_last_kernel_ms(void* ctx, double* ms);
 
 /* Prefill GEMM path (batch_m > 8) of this context's later calls.  Every path
  * runs this library's own kernels except LIBRARY.  AUTO (the default), by
- * measured speed: g64 weights with bf16 activations decode inside the MFMA
- * loop -- the fused kernel up to batch_m 64, the 128 x 128 tile kernel from
- * 128 to 2047 (and beyond when cols > rows); cb4 weights with bf16
+ * measured speed: every kind takes the few-token MFMA kernels up to batch_m
+ * 16, and to 32 or 64 by kind and size; above, g64 weights with bf16
+ * activations decode inside the MFMA loop -- the fused kernel up to batch_m 64,
+ * the 128 x 128 tile kernel from 128 to 767 (1023 when cols > rows); cb4 weights with bf16
  * activations take the cb4 tile kernel described under FUSED from batch_m 128
  * to 511 when the tensor is eligible for it; Q8_0 (and Q4_0) weights with
  * bf16 activations and batch_m <= 128 take the fused kernel; every other call

@@ -15,7 +15,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libvxt_hip.so")
-SOURCES = ["vxt_hip.hip", "gemv.hip", "gemv_q8.hip", "gemv_q8p.hip", "gemv_q40.hip", "gemv_cb4.hip", "gemv_g64.hip", "gemm_panel.hip", "gemm_fused.hip", "gemm_tile.hip", "gemm_dense.hip", "gemm_dense3.hip",
+SOURCES = ["vxt_hip.hip", "gemv.hip", "gemv_q8.hip", "gemv_q8p.hip", "gemv_q40.hip", "gemv_cb4.hip", "gemv_g64.hip", "gemm_panel.hip", "gemm_fused.hip", "gemm_skinny.hip", "gemm_skinny_cb4.hip", "gemm_skinny_g64.hip",
+           "gemm_skinny_q40.hip", "gemm_skinny_q8.hip", "gemm_tile.hip", "gemm_dense.hip", "gemm_dense3.hip",
            "blas_plugin.cpp", "dequant.hip", "greedy.hip", "probe.hip", "ffn.hip", "attn.hip", "archive.cpp"]
 LIBS = ["-ldl"]
 
@@ -45,7 +46,8 @@ FLAGS = [
 # Q8 GEMM (gemm_fused.hip; Q8 M = 128 graph-timed 102 -> 114 and 106 -> 119
 # TFLOP/s on the same box, the g64 instantiations unchanged).
 _VGPR_MFMA = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
-FILE_FLAGS = {"gemv_q8p.hip": _VGPR_MFMA, "gemm_fused.hip": _VGPR_MFMA}
+FILE_FLAGS = {"gemv_q8p.hip": _VGPR_MFMA, "gemm_fused.hip": _VGPR_MFMA,
+              **{f"gemm_skinny_{k}.hip": _VGPR_MFMA for k in ("cb4", "g64", "q40", "q8")}}
 
 
 def _compile(src: str, obj: str, verbose: bool) -> None:

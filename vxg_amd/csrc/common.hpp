@@ -130,6 +130,18 @@ struct NormIn {
   float eps;
 };
 
+// A call of the few-token MFMA kernels (gemm_skinny_impl.hpp): x [M][cols]
+// (x_vec: rows of whole aligned 16-byte pieces), y [M][rows], or with glu the
+// gated activation of [gate; up] into y [M][y_stride].
+struct SkinnyArgs {
+  const void* x;
+  void* y;
+  uint32_t M, x_vec, y_bf16;
+  uint32_t glu, n_ff, y_stride, gelu;
+  uint32_t skip_zero;   // cb4: zero-scale groups are skipped (gemv_cpu, codebook.rs:384-386), not multiplied (gemm_cpu)
+  uint32_t kslice;   // columns of one K range (a multiple of 1024): range z's fp32 sums are y + z * M * rows
+};
+
 // One layer's Q8_0 KV cache (the planes of VxtKvQ8Cache): row t holds
 // position t, n_kv * hd int8 values and n_kv * hd / 32 f16 scales per plane.
 struct KvQ8Dev {

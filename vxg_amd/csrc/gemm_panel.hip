@@ -1093,7 +1093,8 @@ size_t gemm_tile_cb4_workspace_bytes(const DevTensor& t, uint32_t m);
 hipError_t launch_gemm_tile_cb4(const DevTensor& t, const uint16_t* x, uint32_t m, void* y, bool y_bf16, void* ws,
                                 size_t ws_bytes, hipStream_t s);
 
-// Path choice, unless the caller pins one (every path runs every kind):
+// Path choice above the few-token range, unless the caller pins one (every
+// path runs every kind):
 //   * g64 weights, bf16 activations: the fused kernel up to batch 64; the
 //     decode-in-registers tile kernel (gemm_tile.hip) from batch 128 to 767
 //     (to 1023 when K > N); the two-phase path otherwise;
@@ -1131,9 +1132,15 @@ constexpr uint32_t kTileMaxMTall = 1024;   // exclusive, K > N
 constexpr uint32_t kCb4TileMaxM = 512;      // exclusive
 constexpr uint32_t kCb4TileMaxMWide = 256;  // exclusive, K < N
 
+uint32_t skinny_max_m(bool x_bf16);
+size_t skinny_workspace_bytes(const DevTensor& t, uint32_t m, bool x_bf16);
+hipError_t launch_skinny(const DevTensor& t, const void* x, bool x_bf16, uint32_t m, void* y, bool y_bf16, void* ws,
+                         hipStream_t s);
+
 enum class Path { Fused, Tile, TileCb4, Panel };
 
-static Path choose_path(const DevTensor& t, uint32_t m, bool x_bf16, int mode) {
+// The path of a call above the few-token range (or pinned).
+static Path general_path(const DevTensor& t, uint32_t m, bool x_bf16, int mode) {
   if (mode == kGemmPanel || mode == kGemmLibrary) return Path::Panel;
   const bool tile_ok = gemm_tile_supported(t, x_bf16);
   const bool fused_ok = gemm_fused_supported(t, x_bf16);
@@ -1161,8 +1168,8 @@ static bool library_path(int mode) { return mode == kGemmLibrary; }
 // (the tile path keeps its exponents in its own block).
 static size_t xe_bytes(uint32_t m) { return gp::al256((size_t)m * 4); }
 
-size_t gemm_workspace_bytes(const DevTensor& t, uint32_t m, bool x_bf16, int mode) {
-  switch (choose_path(t, m, x_bf16, mode)) {
+static size_t path_workspace_bytes(Path path, const DevTensor& t, uint32_t m, bool x_bf16, int mode) {
+  switch (path) {
     case Path::Tile: return gemm_tile_workspace_bytes(t, m);
     case Path::TileCb4: return gemm_tile_cb4_workspace_bytes(t, m);
     case Path::Fused: return xe_bytes(m) + gemm_fused_workspace_bytes(t, m);
@@ -1172,10 +1179,53 @@ size_t gemm_workspace_bytes(const DevTensor& t, uint32_t m, bool x_bf16, int mod
   return xe_bytes(m) + pl.panel_bytes + pl.a_bytes + pl.partial_bytes;
 }
 
+// The few-token kernels (gemm_skinny.hip) take a call in AUTO up to 16 tokens
+// always, and up to 32 and 64 while each weight's decode, repeated for every
+// 32 tokens, is cheaper than a panel, as measured by kind (whole call, us,
+// this against the general path; K -> N):
+//   M = 17..32: cb4, Q4_0 always (32 tokens 2048 -> 6144 15.7 / 11.6 against
+//   36.0 / 29.7, 2048 -> 151936 238 / 194 against 858 / 526); g64 and Q8_0 up
+//   to 34 M weights, Q8_0 also K <= 4096 (g64 / Q8_0 2048 -> 16384 19.1 / 17.5
+//   against 21.2 / 19.0; 8192 -> 4096 23.2 / 22.3 against 23.4 / 19.0;
+//   2048 -> 151936 170 / 156 against 116 / 142);
+//   M = 33..64: cb4 up to 34 M weights and K <= 4096 (2048 -> 16384 52 against
+//   66; 6144 -> 2048 40 against 36), Q4_0 up to 24 M (4096 -> 4096 24 against
+//   35; 8192 -> 4096 46 against 39), g64 up to 13 M (6144 -> 2048 21.7 against
+//   23.1; 2048 -> 16384 38 against 28), Q8_0 up to 8 M (2048 -> 2048 8.9 against
+//   11.7; 4096 -> 4096 20.4 against 19.1).
+bool skinny_takes(const DevTensor& t, uint32_t m, bool x_bf16) {
+  if (m <= 16) return true;
+  if (m > skinny_max_m(x_bf16)) return false;
+  const size_t w = (size_t)t.cols * t.rows, M1 = 1000 * 1000;
+  if (m <= 32) {
+    if (t.kind == KIND_Q8) return w <= 34 * M1 && t.cols <= 4096;
+    return t.kind != KIND_G64 || w <= 34 * M1;
+  }
+  switch (t.kind) {
+    case KIND_CB4: return w <= 34 * M1 && t.cols <= 4096;
+    case KIND_Q40: return w <= 24 * M1;
+    case KIND_G64: return w <= 13 * M1;
+    default: return w <= 8 * M1;
+  }
+}
+
+static bool takes_skinny(const DevTensor& t, uint32_t m, bool x_bf16, int mode, size_t general_bytes) {
+  return (mode == kGemmAuto || mode == kGemmAutoOwn) && skinny_takes(t, m, x_bf16) &&
+         skinny_workspace_bytes(t, m, x_bf16) <= general_bytes;
+}
+
+// The general path's workspace, also for a call that the few-token kernels
+// take (they need less): which calls fit a capture, or the allocation-free
+// entry point's scratch, does not depend on that choice.
+size_t gemm_workspace_bytes(const DevTensor& t, uint32_t m, bool x_bf16, int mode) {
+  return path_workspace_bytes(general_path(t, m, x_bf16, mode), t, m, x_bf16, mode);
+}
+
 hipError_t launch_gemm(const DevTensor& t, const void* x, bool x_bf16, uint32_t m, void* y, bool y_bf16, void* ws,
                        size_t ws_bytes, hipStream_t s, int mode) {
   if (m == 0 || (size_t)m * t.rows > (size_t)1 << 40) return hipErrorInvalidValue;
-  const Path path = choose_path(t, m, x_bf16, mode);
+  const Path path = general_path(t, m, x_bf16, mode);
+  if (takes_skinny(t, m, x_bf16, mode, ws_bytes)) return launch_skinny(t, x, x_bf16, m, y, y_bf16, ws, s);
   if (path == Path::Tile)
     return launch_gemm_tile(t, static_cast<const uint16_t*>(x), m, y, y_bf16, ws, ws_bytes, s);
   if (path == Path::TileCb4)

@@ -1,0 +1,91 @@
+// gemm_skinny.hip -- entry to the few-token MFMA kernels (gemm_skinny_impl.hpp),
+// instantiated by weight kind in gemm_skinny_{cb4,g64,q40,q8}.hip.
+#include "common.hpp"
+
+namespace vxt {
+
+hipError_t launch_skinny_cb4(const DevTensor&, const SkinnyArgs&, bool, hipStream_t);
+hipError_t launch_skinny_g64(const DevTensor&, const SkinnyArgs&, bool, hipStream_t);
+hipError_t launch_skinny_q40(const DevTensor&, const SkinnyArgs&, bool, hipStream_t);
+hipError_t launch_skinny_q8(const DevTensor&, const SkinnyArgs&, bool, hipStream_t);
+
+hipError_t launch_gemm_reduce(const float* partial, uint32_t splits, const float* inv, const int32_t* xe, uint32_t m,
+                              uint32_t n, void* y, bool y_bf16, hipStream_t s);
+
+static hipError_t launch_any(const DevTensor& t, const SkinnyArgs& a, bool x_bf16, hipStream_t s) {
+  switch (t.kind) {
+    case KIND_CB4: return launch_skinny_cb4(t, a, x_bf16, s);
+    case KIND_G64: return launch_skinny_g64(t, a, x_bf16, s);
+    case KIND_Q40: return launch_skinny_q40(t, a, x_bf16, s);
+    case KIND_Q8: return launch_skinny_q8(t, a, x_bf16, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+static SkinnyArgs args(const DevTensor& t, const void* x, bool x_bf16, uint32_t m, void* y, bool y_bf16) {
+  SkinnyArgs a{};
+  a.x = x;
+  a.y = y;
+  a.M = m;
+  const size_t esz = x_bf16 ? 2 : 4;
+  a.x_vec = reinterpret_cast<uintptr_t>(x) % 16 == 0 && t.cols % 8 == 0 && ((size_t)t.cols * esz) % 16 == 0;
+  a.y_bf16 = y_bf16;
+  a.skip_zero = m <= 8;   // batch_m 1..8 is the GEMV, above the GEMM
+  a.kslice = (t.cols + 1023u) / 1024u * 1024u;
+  return a;
+}
+
+// K ranges of a call, each a set of workgroups of its own, summed by the
+// split-K reduction.
+static uint32_t k_slices(const DevTensor& t, uint32_t m, bool x_bf16) {
+  if (!x_bf16 || m <= 8) return 1;
+  return (t.cols + 2047u) / 2048u;
+}
+
+// The most tokens of one call.
+uint32_t skinny_max_m(bool x_bf16) { return x_bf16 ? 64u : 16u; }
+
+size_t skinny_workspace_bytes(const DevTensor& t, uint32_t m, bool x_bf16) {
+  const uint32_t sl = k_slices(t, m, x_bf16);
+  return sl > 1 ? (size_t)sl * m * t.rows * 4 : 0;
+}
+
+hipError_t launch_skinny(const DevTensor& t, const void* x, bool x_bf16, uint32_t m, void* y, bool y_bf16, void* ws,
+                         hipStream_t s) {
+  const uint32_t sl = k_slices(t, m, x_bf16);
+  SkinnyArgs a = args(t, x, x_bf16, m, sl > 1 ? ws : y, sl > 1 ? false : y_bf16);
+  if (sl > 1) a.kslice = 2048;
+  const hipError_t e = launch_any(t, a, x_bf16, s);
+  if (e != hipSuccess || sl == 1) return e;
+  return launch_gemm_reduce(static_cast<const float*>(ws), sl, nullptr, nullptr, m, t.rows, y, y_bf16, s);
+}
+
+// Whether a gated call takes the fused form: up to 8 tokens always (but Q8_0
+// with 3 .. 8 aligned bf16 tokens, whose plain GEMV has kernels of its own: the
+// staged form keeps its sums), above (in AUTO) up to 16, and up to 64 bf16 tokens while K fits one phase range and
+// the decode, repeated for every 32 tokens, stays below the staged form's
+// GEMM, f32 gate and up rows and element-wise pass (32 / 64 tokens, K = 2048,
+// n_ff = 6144, us against the staged form: cb4 27 / 40 against 58 / 59, g64 20
+// / 29 against 25 / 34, Q4_0 22 / 32 against 41 / 40, Q8_0 18 / 26 against 23
+// / 30).
+bool skinny_glu_takes(const DevTensor& t, const void* x, uint32_t m, bool x_bf16, int mode) {
+  if (m <= 8) return t.kind != KIND_Q8 || m == 2 || !args(t, x, x_bf16, m, nullptr, false).x_vec || !x_bf16;
+  if (mode != kGemmAuto && mode != kGemmAutoOwn) return false;
+  if (m <= 16) return true;
+  const size_t w = (size_t)t.cols * t.rows, M1 = 1000 * 1000;
+  return m <= skinny_max_m(x_bf16) && t.cols <= 2048 && w <= (m <= 32 ? 34 : 26) * M1;
+}
+
+// Gated [gate; up] form: act[m][i] = f(gate_i) * up_i for i < rows / 2, zero
+// up to act_stride.
+hipError_t launch_skinny_glu(const DevTensor& t, const void* x, bool x_bf16, uint32_t m, void* act, bool act_bf16,
+                             uint32_t act_stride, bool gelu, hipStream_t s) {
+  SkinnyArgs a = args(t, x, x_bf16, m, act, act_bf16);
+  a.glu = 1;
+  a.n_ff = t.rows / 2;
+  a.y_stride = act_stride;
+  a.gelu = gelu;
+  return launch_any(t, a, x_bf16, s);
+}
+
+}  // namespace vxt

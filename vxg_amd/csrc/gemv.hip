@@ -21,11 +21,18 @@ hipError_t launch_glu_cb4(const DevTensor&, const void*, bool, uint32_t, uint32_
 hipError_t launch_glu_g64(const DevTensor&, const void*, bool, uint32_t, uint32_t, void*, bool, uint32_t, bool,
                           hipStream_t);
 
-// x_vec (x rows 16-byte aligned) is accepted for the ABI layer; the kernels
-// stage activations through LDS or read them element-wise.
+hipError_t launch_skinny(const DevTensor&, const void*, bool, uint32_t, void*, bool, void*, hipStream_t);
+
+// Two tokens and more run on the few-token MFMA kernels, except Q8_0 with
+// aligned bf16 activations (x_vec), whose own kernels stream int8 as fast or
+// faster (2048 x 2048 / 2048 x 6144 / 151936 x 2048 at M = 4: 3.7 / 5.6 / 63
+// us).  M = 4, K x N = 2048 x 6144 / 6144 x 2048 / 2048 x 151936 against the
+// one-FMA-per-weight-per-token kernel before: cb4 22.3 / 19.1 / 543 -> 8.3 /
+// 8.2 / 75 us, g64 20.3 / 18.7 / 459 -> 6.6 / 7.4 / 67, Q4_0 12.4 / 11.4 /
+// 265 -> 6.0 / 7.0 / 61.
 hipError_t launch_gemv(const DevTensor& t, const void* x, bool x_bf16, bool x_vec, uint32_t m, void* y,
                        bool y_bf16, hipStream_t s) {
-  (void)x_vec;
+  if (m >= 2 && (t.kind != KIND_Q8 || !x_bf16 || !x_vec)) return launch_skinny(t, x, x_bf16, m, y, y_bf16, nullptr, s);
   switch (t.kind) {
     case KIND_Q8: return launch_gemv_q8(t, x, x_bf16, m, y, y_bf16, s);
     case KIND_Q40: return launch_gemv_q40(t, x, x_bf16, m, y, y_bf16, s);
@@ -35,7 +42,7 @@ hipError_t launch_gemv(const DevTensor& t, const void* x, bool x_bf16, bool x_ve
   }
 }
 
-// Gated gate/up GEMV (batch_m 1..8): t is [gate; up] with t.rows = 2 * n_ff.
+// Gated gate/up GEMV (one token): t is [gate; up] with t.rows = 2 * n_ff.
 hipError_t launch_gemv_glu(const DevTensor& t, const void* x, bool x_bf16, uint32_t m, void* act, bool act_bf16,
                            uint32_t act_stride, bool gelu, hipStream_t s) {
   const uint32_t n_ff = t.rows / 2;

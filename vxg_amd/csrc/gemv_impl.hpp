@@ -352,8 +352,8 @@ __device__ __forceinline__ void read_x_lds(const uint16_t* s_xn, uint32_t k0, fl
   }
 }
 
-// Kernel: MT tokens (MT in {1,2,4,8}; m >= M_rt are padding), RPW rows per
-// wave, up to S steps per batch.  Gated epilogues take n_ff and the output
+// Kernel: MT tokens (m >= M_rt are padding; more than one token runs on the
+// MFMA kernels of gemm_skinny_impl.hpp), RPW rows per wave, up to S steps per batch.  Gated epilogues take n_ff and the output
 // row stride; the plain epilogue ignores both.  NORM: the norm prologue above
 // (MT = 1, bf16 x staged in dynamic LDS of nsteps * kStep elements).
 // KS > 1 (split K): the workgroup's KS waves share its RPW rows, wave w
@@ -381,7 +381,6 @@ __global__ __launch_bounds__(kWaves * 64) void gemv_kernel(DevTensor t, const vo
   const uint32_t first = KS > 1 ? blockIdx.x * kOut : (blockIdx.x * kWaves + wave) * kOut;
   const uint32_t rows = t.rows, cols = t.cols, kp = t.kp;
   const uint32_t nsteps = (kp + kStep - 1) / kStep;
-  constexpr bool kLateX = MT >= 4;
   uint32_t rr[RPW];
   bool rv[RPW];
   wave_rows<EPI, RPW>(first, rows, n_ff, rr, rv);
@@ -433,15 +432,15 @@ __global__ __launch_bounds__(kWaves * 64) void gemv_kernel(DevTensor t, const vo
   for (uint32_t s0 = KS > 1 ? wave : 0u; s0 < nsteps; s0 += KS > 1 ? (uint32_t)KS : (uint32_t)S) {
     const uint32_t ns = nsteps - s0 < (uint32_t)S ? nsteps - s0 : (uint32_t)S;   // uniform
     // ---- issue: activations, then weights, for every step of the batch
-    XChunk<XBF16> xc[kLateX ? 1 : S][kLateX ? 1 : MT];
+    XChunk<XBF16> xc[S][MT];
     WChunk<KIND> wc[S][RPW];
 #pragma unroll
     for (int s = 0; s < S; ++s) {
-      if (!NORM && !kLateX && (uint32_t)s < ns && x_vec) {
+      if (!NORM && (uint32_t)s < ns && x_vec) {
         const uint32_t k0 = (s0 + s) * kStep + lane * kChunk;
 #pragma unroll
         for (int m = 0; m < MT; ++m)
-          load_x<XBF16>(x, cols, (uint32_t)m < M_rt ? m : 0, k0, xc[kLateX ? 0 : s][kLateX ? 0 : m]);
+          load_x<XBF16>(x, cols, (uint32_t)m < M_rt ? m : 0, k0, xc[s][m]);
       }
     }
 #pragma unroll
@@ -474,13 +473,10 @@ __global__ __launch_bounds__(kWaves * 64) void gemv_kernel(DevTensor t, const vo
       if ((uint32_t)s >= ns) break;
       const uint32_t k0 = (s0 + s) * kStep + lane * kChunk;
       const bool kin = k0 < kp;
-      // Early x: every token unpacked once per step.  Late x (MT >= 4): each
-      // token is loaded and unpacked where it is used, so the registers hold
-      // one token's 32 values at a time.
-      float xv[kLateX ? 1 : MT][kChunk];
+      float xv[MT][kChunk];   // every token unpacked once per step
       if constexpr (NORM) {
         read_x_lds(s_xn, k0, xv[0]);
-      } else if constexpr (!kLateX) {
+      } else {
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
           if (x_vec)
@@ -503,17 +499,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemv_kernel(DevTensor t, const vo
         dequant_chunk<KIND>(wc[s][r], cbase, sl, lane, w);
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
-          const float* xm = xv[kLateX ? 0 : m];
-          if constexpr (kLateX) {
-            const uint32_t mm = (uint32_t)m < M_rt ? m : 0;
-            if (x_vec) {
-              XChunk<XBF16> c;
-              load_x<XBF16>(x, cols, mm, k0, c);
-              unpack_x<XBF16>(c, xv[0]);
-            } else {
-              load_x_scalar<XBF16>(x, cols, mm, k0, xv[0]);
-            }
-          }
+          const float* xm = xv[m];
           float p0 = 0.0f, p1 = 0.0f;
 #pragma unroll
           for (int j = 0; j < kChunk; j += 2) {
@@ -1847,7 +1833,7 @@ template <uint32_t KIND, int MT, int RPW, bool XBF16>
 hipError_t launch_s(const DevTensor& t, const void* x, uint32_t m, void* y, bool y_bf16, hipStream_t s) {
   const uint32_t nsteps = (t.kp + kStep - 1) / kStep;
   if (nsteps == 1) return launch_t<KIND, MT, RPW, 1, XBF16>(t, x, m, y, y_bf16, s);
-  if (nsteps == 3 && MT <= 2) return launch_t<KIND, MT, RPW, 3, XBF16>(t, x, m, y, y_bf16, s);
+  if (nsteps == 3) return launch_t<KIND, MT, RPW, 3, XBF16>(t, x, m, y, y_bf16, s);
   return launch_t<KIND, MT, RPW, 2, XBF16>(t, x, m, y, y_bf16, s);
 }
 
@@ -2027,19 +2013,11 @@ hipError_t launch_kind(const DevTensor& t, const void* x, bool x_bf16, uint32_t 
     if (t.rows >= 4096) return launch_r<KIND, 1, 2>(t, x, x_bf16, m, y, y_bf16, s);
     return launch_r<KIND, 1, 1>(t, x, x_bf16, m, y, y_bf16, s);
   }
-  if (m == 2) {
-    if (t.rows >= 65536) return launch_r<KIND, 2, 2>(t, x, x_bf16, m, y, y_bf16, s);
-    return launch_r<KIND, 2, 1>(t, x, x_bf16, m, y, y_bf16, s);
-  }
-  if (m <= 4) return launch_r<KIND, 4, 1>(t, x, x_bf16, m, y, y_bf16, s);
-  if (m <= 8) return launch_r<KIND, 8, 1>(t, x, x_bf16, m, y, y_bf16, s);
   return hipErrorInvalidValue;
 }
 
-// Gated gate/up GEMV: one output (a gate row and its up row) per wave, the
-// generic kernel for every kind, M = 1 or 2 (the gate and up accumulators of
-// four or more tokens do not fit in registers without spilling; the caller
-// runs those as a plain GEMV and an element-wise activation pass).
+// Gated gate/up GEMV of one token: one output (a gate row and its up row) per
+// wave, the generic kernel for every kind (more tokens: gemm_skinny.hip).
 template <uint32_t KIND, int MT, int S, bool XBF16, int EPI>
 hipError_t launch_glu_t(const DevTensor& t, const void* x, uint32_t m, uint32_t n_ff, void* y, bool y_bf16,
                         uint32_t y_stride, hipStream_t s) {
@@ -2058,7 +2036,7 @@ hipError_t launch_glu_s(const DevTensor& t, const void* x, uint32_t m, uint32_t 
                         uint32_t y_stride, hipStream_t s) {
   const uint32_t nsteps = (t.kp + kStep - 1) / kStep;
   if (nsteps == 1) return launch_glu_t<KIND, MT, 1, XBF16, EPI>(t, x, m, n_ff, y, y_bf16, y_stride, s);
-  if (nsteps == 3 && MT <= 2) return launch_glu_t<KIND, MT, 3, XBF16, EPI>(t, x, m, n_ff, y, y_bf16, y_stride, s);
+  if (nsteps == 3) return launch_glu_t<KIND, MT, 3, XBF16, EPI>(t, x, m, n_ff, y, y_bf16, y_stride, s);
   return launch_glu_t<KIND, MT, 2, XBF16, EPI>(t, x, m, n_ff, y, y_bf16, y_stride, s);
 }
 
@@ -2097,7 +2075,6 @@ hipError_t launch_glu_m(const DevTensor& t, const void* x, bool x_bf16, uint32_t
     if (m == 1 && try_glu_cb4_m1<EPI>(t, x, x_bf16, n_ff, y, y_bf16, y_stride, s, &e)) return e;
   }
   if (m == 1) return launch_glu_x<KIND, 1, EPI>(t, x, x_bf16, m, n_ff, y, y_bf16, y_stride, s);
-  if (m == 2) return launch_glu_x<KIND, 2, EPI>(t, x, x_bf16, m, n_ff, y, y_bf16, y_stride, s);
   return hipErrorInvalidValue;
 }
 

@@ -57,6 +57,9 @@ hipError_t launch_attn_prefill(const KvQ8Dev& c, const float* q, const float* ga
 size_t greedy_state_bytes();
 hipError_t launch_greedy(const float* logits, uint32_t n, void* state, uint32_t* out, hipStream_t s);
 hipError_t launch_read_probe(const void* p, size_t bytes, uint32_t* sink, uint32_t key, hipStream_t s);
+bool skinny_glu_takes(const DevTensor& t, const void* x, uint32_t m, bool x_bf16, int mode);
+hipError_t launch_skinny_glu(const DevTensor& t, const void* x, bool x_bf16, uint32_t m, void* act, bool act_bf16,
+                             uint32_t act_stride, bool gelu, hipStream_t s);
 void blas_acquire_device(int dev);
 void blas_release_device(int dev);
 }  // namespace vxt
@@ -928,22 +931,24 @@ int vxt_hip_ffn_glu_dev(void* ctx, void* tensor, const void* x, uint32_t x_dtype
     hipStream_t s = static_cast<hipStream_t>(stream);
     const DevTensor d = t->dev();
     hipError_t e;
-    if (batch_m <= 2) {
-      e = vxt::launch_gemv_glu(d, x, xb, batch_m, act, ab, act_stride, gelu, s);
+    if (batch_m == 1) {
+      e = vxt::launch_gemv_glu(d, x, xb, 1, act, ab, act_stride, gelu, s);
     } else {
-      // Gate and up rows into f32 staging after the GEMM's own workspace,
-      // then the element-wise activation.
+      // The workspace of the staged form: the GEMM's own, then gate and up
+      // rows in f32.  The fused few-token form uses none of it; what a call
+      // reserves does not depend on the form.
       const size_t gemm_ws =
           batch_m > 8 ? (vxt::gemm_workspace_bytes(d, batch_m, xb, c->gemm_mode) + 255) / 256 * 256 : 0;
       const size_t stage = (size_t)batch_m * t->rows * sizeof(float);
-      ensure_ws(c, gemm_ws + stage, s);
-      float* gu = reinterpret_cast<float*>(static_cast<char*>(c->ws) + gemm_ws);
-      if (batch_m <= 8) {
-        e = vxt::launch_gemv(d, x, xb, false, batch_m, gu, false, s);
+      if (batch_m > 2) ensure_ws(c, gemm_ws + stage, s);
+      if (vxt::skinny_glu_takes(d, x, batch_m, xb, c->gemm_mode)) {
+        e = vxt::launch_skinny_glu(d, x, xb, batch_m, act, ab, act_stride, gelu, s);
       } else {
-        e = vxt::launch_gemm(d, x, xb, batch_m, gu, false, c->ws, gemm_ws, s, c->gemm_mode);
+        float* gu = reinterpret_cast<float*>(static_cast<char*>(c->ws) + gemm_ws);
+        e = batch_m <= 8 ? vxt::launch_gemv(d, x, xb, true, batch_m, gu, false, s)
+                         : vxt::launch_gemm(d, x, xb, batch_m, gu, false, c->ws, gemm_ws, s, c->gemm_mode);
+        if (e == hipSuccess) e = vxt::launch_glu_act(gu, batch_m, n_ff, gelu, act, ab, act_stride, s);
       }
-      if (e == hipSuccess) e = vxt::launch_glu_act(gu, batch_m, n_ff, gelu, act, ab, act_stride, s);
     }
     if (e == hipErrorNotSupported) fail(VXT_E_UNSUPPORTED, "batch_m > 8 GEMM not available for this tensor");
     if (e != hipSuccess) fail(VXT_E_DEVICE, std::string("gated FFN launch failed: ") + hipGetErrorString(e));
