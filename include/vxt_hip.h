@@ -560,7 +560,7 @@ VXT_API int vxt_hip_last_kernel_ms(void* ctx, double* ms);
  * measured speed: every kind takes the few-token MFMA kernels up to batch_m
  * 16, and to 32 or 64 by kind and size; above, g64 weights with bf16
  * activations decode inside the MFMA loop -- the fused kernel up to batch_m 64,
- * the 128 x 128 tile kernel from 128 to 767 (1023 when cols > rows); cb4 weights with bf16
+ * the 128 x 128 tile kernel above, to 767 (1023 when cols > rows); cb4 weights with bf16
  * activations take the cb4 tile kernel described under FUSED from batch_m 128
  * to 511 when the tensor is eligible for it; Q8_0 (and Q4_0) weights with
  * bf16 activations and batch_m <= 128 take the fused kernel; every other call

@@ -258,3 +258,16 @@ def test_cb4_tile_kernel_residual_cap(eng):
     e = check(eng, over, 200, engine.GEMM_FUSED, seed=5)   # pinned: falls back to the two-phase path too
     assert np.array_equal(c.view(np.uint32), d.view(np.uint32))
     assert np.array_equal(e.view(np.uint32), d.view(np.uint32))
+
+
+# Grids kept within one workgroup per CU (96 tiles in two K slices, 40 in five or
+# six, 144 in one), the shortest batches of the automatic choice (65 up), and
+# ragged partial sums whose rows and columns end inside a tile.
+@pytest.mark.parametrize("M,N,K", [(65, 1000, 4096), (127, 2100, 1030), (200, 6144, 512), (130, 2500, 2048),
+                                   (300, 6100, 576)])
+def test_tile_kernel_one_round_grids(eng, M, N, K):
+    print(f"tile one-round grid M={M} N={N} K={K}", flush=True)
+    a = check(eng, synth.make_g64(N, K, seed=M + N), M, engine.GEMM_AUTO, seed=K)
+    b = check(eng, synth.make_g64(N, K, seed=M + N), M, engine.GEMM_FUSED, seed=K)
+    assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    check(eng, make("cb4", N, K, seed=M + N), M, engine.GEMM_FUSED, seed=K)

@@ -65,6 +65,19 @@ __device__ __forceinline__ uint4 load_nt16(const void* p) {
   return make_uint4(v.x, v.y, v.z, v.w);
 }
 
+// Stores of a ragged output tile without a branch each: a raw buffer over
+// `rows` whole rows of n floats from `base` (rows * n * 4 < 2^31); the
+// hardware drops a store past its end, i.e. of a row >= rows.  A lane whose
+// column is past n starts at kDropped, which no row brings back in range.
+constexpr uint32_t kDropped = 0x80000000u;
+__device__ __forceinline__ bool rows_fit(uint32_t rows, uint32_t n) { return (uint64_t)rows * n * 4u < kDropped; }
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_rsrc(float* base, uint32_t rows, uint32_t n) {
+  return __builtin_amdgcn_make_buffer_rsrc(base, (short)0, (int)(rows * n * 4u), 0x00020000);
+}
+__device__ __forceinline__ void rows_store(__amdgpu_buffer_rsrc_t r, uint32_t off, float v) {
+  __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, (int)off, 0, 0);
+}
+
 // ---- conversions ---------------------------------------------------------
 
 // Exact f16 -> f32 in integer arithmetic: the reference's rule

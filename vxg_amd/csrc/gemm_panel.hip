@@ -1096,15 +1096,17 @@ hipError_t launch_gemm_tile_cb4(const DevTensor& t, const uint16_t* x, uint32_t 
 // Path choice above the few-token range, unless the caller pins one (every
 // path runs every kind):
 //   * g64 weights, bf16 activations: the fused kernel up to batch 64; the
-//     decode-in-registers tile kernel (gemm_tile.hip) from batch 128 to 767
-//     (to 1023 when K > N); the two-phase path otherwise;
+//     decode-in-registers tile kernel (gemm_tile.hip) above, to 767 (to 1023
+//     when K > N); the two-phase path otherwise;
 //   * cb4 weights, bf16 activations, within the tile kernel's limits
 //     (gemm_tile_cb4_supported): its decode-in-loop tile kernel from batch
 //     128 to 511, to 255 when K < N (M = 128 / 256: 96 / 84 and 137 / 145
 //     TFLOP/s against the two-phase path's 81 / 77 and 121 / 131; at M = 64
 //     and 512 the two-phase path is ahead; with the two-phase planes in 1 KB
 //     pieces, at 2048 -> 6144 M = 256 / 384: 133 / 146 against 149 / 172,
-//     at 6144 -> 2048 148 / 169 against 143 / 160);
+//     at 6144 -> 2048 148 / 169 against 143 / 160).  Not below 128, where it
+//     would be ahead (2048 -> 12288 M = 100: 43 against 52 us): an Inf activation
+//     makes its whole row NaN there, and +-Inf on the two-phase path;
 //   * Q8 weights, bf16 activations: the fused kernel up to batch 128, and
 //     up to 511 when K >= N (M = 256 / 384: 196 / 212 TFLOP/s against
 //     171 / 182 two-phase at 6144 -> 2048, 91 / 126 against 81 / 106 at
@@ -1114,8 +1116,9 @@ hipError_t launch_gemm_tile_cb4(const DevTensor& t, const uint16_t* x, uint32_t 
 // The vendor dense GEMM runs only when pinned (kGemmLibrary), as a
 // comparison.  Measured on MI355X (whole call, graph of 100 calls, TFLOP/s,
 // K x N = 2048 x 6144 / 6144 x 2048):
-//   g64 M = 64: fused 73 / 61, two-phase 68 / 61; M = 96: tile 82, two-phase
-//   89 (2048 x 6144); M = 128: tile 134 / 118, two-phase 115 / 107; M = 512:
+//   g64 M = 64: fused 73 / 61, two-phase 68 / 61; M = 72: tile 95, two-phase
+//   78 (2048 x 6144); M = 100: tile 214, two-phase 161 (2048 x 12288); M = 128:
+//   tile 134 / 118, two-phase 115 / 107; M = 512:
 //   tile 407 / 350, two-phase 300 / 325; with the two-phase planes in 1 KB
 //   pieces: M = 512: tile 409 / 358, two-phase 418 / 321; M = 768: tile
 //   378 / 396, two-phase 457 / 384; M = 1024: tile 484 / 463, two-phase
@@ -1126,7 +1129,7 @@ hipError_t launch_gemm_tile_cb4(const DevTensor& t, const uint16_t* x, uint32_t 
 constexpr uint32_t kFusedMaxM = 128;
 constexpr uint32_t kQ8FusedMaxMTall = 512;   // exclusive, K >= N
 constexpr uint32_t kG64FusedMaxM = 64;
-constexpr uint32_t kTileMinM = 128;
+constexpr uint32_t kCb4TileMinM = 128;
 constexpr uint32_t kTileMaxM = 768;        // exclusive
 constexpr uint32_t kTileMaxMTall = 1024;   // exclusive, K > N
 constexpr uint32_t kCb4TileMaxM = 512;      // exclusive
@@ -1149,12 +1152,12 @@ static Path general_path(const DevTensor& t, uint32_t m, bool x_bf16, int mode) 
     if (tile_ok && m > kG64FusedMaxM) return Path::Tile;
     return fused_ok ? Path::Fused : Path::Panel;
   }
-  if (t.kind == KIND_CB4 && m >= kTileMinM && m < (t.cols < t.rows ? kCb4TileMaxMWide : kCb4TileMaxM) &&
+  if (t.kind == KIND_CB4 && m >= kCb4TileMinM && m < (t.cols < t.rows ? kCb4TileMaxMWide : kCb4TileMaxM) &&
       gemm_tile_cb4_supported(t, x_bf16))
     return Path::TileCb4;
   if (t.kind == KIND_G64 && x_bf16) {
     if (fused_ok && m <= kG64FusedMaxM) return Path::Fused;
-    if (tile_ok && m >= kTileMinM && m < (t.cols > t.rows ? kTileMaxMTall : kTileMaxM)) return Path::Tile;
+    if (tile_ok && m > kG64FusedMaxM && m < (t.cols > t.rows ? kTileMaxMTall : kTileMaxM)) return Path::Tile;
     return Path::Panel;
   }
   if (fused_ok && (m <= kFusedMaxM || (t.kind == KIND_Q8 && t.cols >= t.rows && m < kQ8FusedMaxMTall)))
@@ -1218,7 +1221,12 @@ static bool takes_skinny(const DevTensor& t, uint32_t m, bool x_bf16, int mode, 
 // take (they need less): which calls fit a capture, or the allocation-free
 // entry point's scratch, does not depend on that choice.
 size_t gemm_workspace_bytes(const DevTensor& t, uint32_t m, bool x_bf16, int mode) {
-  return path_workspace_bytes(general_path(t, m, x_bf16, mode), t, m, x_bf16, mode);
+  const Path path = general_path(t, m, x_bf16, mode);
+  size_t n = path_workspace_bytes(path, t, m, x_bf16, mode);
+  // below 128 tokens the g64 tile kernel needs less than the two-phase path: the same holds there
+  if (path == Path::Tile && m < 128 && mode != kGemmFused)
+    n = std::max(n, path_workspace_bytes(Path::Panel, t, m, x_bf16, mode));
+  return n;
 }
 
 hipError_t launch_gemm(const DevTensor& t, const void* x, bool x_bf16, uint32_t m, void* y, bool y_bf16, void* ws,

@@ -500,6 +500,13 @@ __global__ __launch_bounds__(NT * KW, KW == 1 ? 2 : 1) void tile_kernel(DevTenso
         for (int f = 0; f < 4; ++f)
 #pragma unroll
           for (int r = 0; r < 16; ++r) pp[(size_t)row_of(f, r) * N_] = acc[f][r];
+      } else if (rows_fit(BM, N_)) {   // ragged (g64 M = 100, 2048 -> 12288: 29.1 us, with a branch per output 32.1)
+        const auto rs = rows_rsrc(partial + ((size_t)blockIdx.y * M + m0) * N_, std::min(M - m0, (uint32_t)BM), N_);
+        const uint32_t c0 = ncol < N_ ? ncol * 4u : kDropped;
+#pragma unroll
+        for (int f = 0; f < 4; ++f)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) rows_store(rs, c0 + row_of(f, r) * N_ * 4u, acc[f][r]);
       } else {
 #pragma unroll
         for (int f = 0; f < 4; ++f)
@@ -1002,6 +1009,13 @@ __global__ __launch_bounds__(NT, 1) void tile_cb4_kernel(DevTensor t, const uint
       for (int f = 0; f < 4; ++f)
 #pragma unroll
         for (int r = 0; r < 16; ++r) pp[(size_t)row_of(f, r) * N_] = ldexpf(value(f, r), -er);
+    } else if (rows_fit(BM, N_)) {   // ragged
+      const auto rs = rows_rsrc(partial + ((size_t)blockIdx.y * M + m0) * N_, std::min(M - m0, (uint32_t)BM), N_);
+      const uint32_t c0 = ncol < N_ ? ncol * 4u : kDropped;
+#pragma unroll
+      for (int f = 0; f < 4; ++f)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) rows_store(rs, c0 + row_of(f, r) * N_ * 4u, ldexpf(value(f, r), -er));
     } else {
 #pragma unroll
       for (int f = 0; f < 4; ++f)
@@ -1049,7 +1063,11 @@ inline size_t al256(size_t v) { return (v + 255) & ~size_t(255); }
 // tiles on, one K-way; below, K split across workgroups until the grid has
 // about 256 workgroups, with >= 4 tiles per slice and at most 16 MB of
 // partial sums, and two K-ways (8 waves, one workgroup per CU) unless that
-// takes more than 4 slices.
+// takes more than 4 slices.  Where one workgroup fills a CU the grid stays
+// within the 256 CUs: a slice more put 288 workgroups on them, two rounds of
+// two thirds (M = 200, 2048 -> 6144, 96 tiles, whole call: g64 32.8 -> 24.6 us, cb4 59.2 ->
+// 42.8).  The workspace is sized for the slice count rounded up, the most a
+// call of the shape has needed.
 constexpr size_t kMaxPartialBytes = (size_t)16 << 20;
 
 inline Plan plan(const DevTensor& t, uint32_t m) {
@@ -1068,6 +1086,12 @@ inline Plan plan(const DevTensor& t, uint32_t m) {
   }
   p.kps = (ktt + splits - 1) / splits;
   p.splits = (ktt + p.kps - 1) / p.kps;
+  const uint32_t reserve = p.splits;
+  if (p.kw == 2 && p.splits <= 4) {
+    splits = std::min(splits, std::max(1u, 256u / tiles));
+    p.kps = (ktt + splits - 1) / splits;
+    p.splits = (ktt + p.kps - 1) / p.kps;
+  }
   // With more than 4 K slices each way would walk only a few tiles: one
   // K-way per workgroup is then faster (M = 128: 11.9 against 12.7 us at
   // 6144 x 2048, 12.8 against 14.2 us at 2048 x 6144).
@@ -1075,7 +1099,7 @@ inline Plan plan(const DevTensor& t, uint32_t m) {
   p.xe_off = 0;
   p.xh_off = al256((size_t)m * 4);
   p.partial_off = p.xh_off + al256((size_t)m * t.kp * 2);
-  p.bytes = p.partial_off + (p.splits > 1 ? al256((size_t)p.splits * m * t.rows * 4) : 0);
+  p.bytes = p.partial_off + (reserve > 1 ? al256((size_t)reserve * m * t.rows * 4) : 0);
   return p;
 }
 
@@ -1107,11 +1131,14 @@ inline Plan plan_cb4(const DevTensor& t, uint32_t m) {
   splits = std::min<uint32_t>(splits, std::max<uint32_t>(1u, ktt / 2));
   splits = (uint32_t)std::min<size_t>(splits, std::max<size_t>(1, kMaxPartialBytes / slice_bytes));
   p.kps = (ktt + splits - 1) / splits;
+  const uint32_t reserve = (ktt + p.kps - 1) / p.kps;
+  splits = std::min(splits, std::max(1u, 256u / tiles));
+  p.kps = (ktt + splits - 1) / splits;
   p.splits = (ktt + p.kps - 1) / p.kps;
   p.xe_off = 0;
   p.xh_off = al256((size_t)m * 4);
   p.partial_off = p.xh_off + al256((size_t)m * t.kp * 2);
-  p.bytes = p.partial_off + (p.splits > 1 ? al256((size_t)p.splits * m * t.rows * 4) : 0);
+  p.bytes = p.partial_off + (reserve > 1 ? al256((size_t)reserve * m * t.rows * 4) : 0);
   return p;
 }
 
