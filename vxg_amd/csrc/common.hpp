@@ -50,6 +50,9 @@ struct DevTensor {
 // first call for a shape allocates descriptors).
 enum GemmMode : int { kGemmAuto = 0, kGemmPanel = 1, kGemmFused = 2, kGemmLibrary = 3, kGemmAutoOwn = 4 };
 
+// Bytes of the scratch array of the allocation-free matmul entry point.
+constexpr size_t kNoAllocScratch = (size_t)32 << 20;
+
 // Centroid table serving `row` (rows of up to 3 concatenated sub-matrices).
 __device__ __forceinline__ uint32_t cent_table(const DevTensor& t, uint32_t row) {
   return (uint32_t)(row >= t.split0) + (uint32_t)(row >= t.split1);
@@ -153,6 +156,19 @@ struct SkinnyArgs {
   uint32_t glu, n_ff, y_stride, gelu;
   uint32_t skip_zero;   // cb4: zero-scale groups are skipped (gemv_cpu, codebook.rs:384-386), not multiplied (gemm_cpu)
   uint32_t kslice;   // columns of one K range (a multiple of 1024): range z's fp32 sums are y + z * M * rows
+};
+
+// A call of the large-tile dense kernel (gemm_dense3.hip).
+struct D3Args {
+  const uint16_t *ah, *al;   // activation planes; al null for bf16 activations
+  const uint16_t *bh, *bl;
+  const float *dsc, *inv;
+  uint32_t m, n, kp;
+  void* y;
+  bool y_bf16;
+  float* partial;
+  uint32_t splits, kt_per_split;
+  const int32_t* xe;
 };
 
 // One layer's Q8_0 KV cache (the planes of VxtKvQ8Cache): row t holds

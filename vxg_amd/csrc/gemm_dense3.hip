@@ -92,28 +92,32 @@ __device__ __forceinline__ void static_for(F&& f) {
 }
 
 // 4-wave workgroups of 2 x 2-fragment waves (128 x 128 tiles) run two per
-// CU (the LDS budget halves); every other shape one per CU.
-constexpr int occupancy(int wm, int wn, int nw) { return (nw == 4 && wm == 2 && wn == 2) ? 2 : 1; }
+// CU (the LDS budget halves); every other shape, and those with split
+// activations (twice the A stages), one per CU.
+constexpr int occupancy(int wm, int wn, int nw, bool sa) { return (nw == 4 && wm == 2 && wn == 2 && !sa) ? 2 : 1; }
 
-// NW waves per workgroup in NW / 2 x 2 (wave rows x wave columns).
-template <int WM, int WN, int MODE, int NW = 4>
+// NW waves per workgroup in NW / 2 x 2 (wave rows x wave columns).  SA: split
+// activations (f32 x = hi + lo * 2^-11, two planes).
+template <int WM, int WN, int MODE, int NW, bool SA>
 struct Cfg {
   static constexpr int NT = 64 * NW;
   static constexpr int BM = 32 * WM * (NW / 2), BN = 64 * WN;
   static constexpr bool LO = MODE == kHiLo, QB = MODE == kQBlock;
   static constexpr int A_BYTES = BM * 64, B_BYTES = BN * 64;   // one stage of one operand
   static constexpr int D_BYTES = QB ? BN * 4 : 16;             // Q8 block: the tile's scales
-  static constexpr int STAGE = A_BYTES + B_BYTES * (LO ? 2 : 1) + (QB ? D_BYTES : 0);
-  static constexpr int OCC = occupancy(WM, WN, NW);
+  static constexpr int STAGE = A_BYTES * (SA ? 2 : 1) + B_BYTES * (LO ? 2 : 1) + (QB ? D_BYTES : 0);
+  static constexpr int OCC = occupancy(WM, WN, NW, SA);
   // Q8 block mode alternates two scale register sets by stage parity (tile t
   // uses set t & 1 from stage t mod NS), which needs an even stage count.
   static constexpr int NS0 = std::min(5, (160 * 1024 / OCC - 2048) / STAGE);
   static constexpr int NS = QB ? NS0 & ~1 : NS0;
   static constexpr int NA = BM / (16 * NW), NB = BN / (16 * NW), NL = LO ? NB : 0;   // 1 KB loads per wave per tile
   static constexpr int ND = QB ? 1 : 0;   // one 4-byte-per-lane scale load per wave per tile
-  static constexpr int NLD = NA + NB + NL + ND;
-  static constexpr int NR = WM + WN + (LO ? WN : 0);   // fragment reads per step
-  static constexpr int NM = WM * WN * (LO ? 2 : 1);    // MFMAs per step
+  static constexpr int NS_A = SA ? NA : 0;
+  static constexpr int NLD = NA + NS_A + NB + NL + ND;
+  static constexpr int NR = WM * (SA ? 2 : 1) + WN * (LO ? 2 : 1);   // fragment reads per step
+  static constexpr int TERMS = 1 + (LO ? 1 : 0) + (SA ? 1 : 0);       // MFMAs per fragment product
+  static constexpr int NM = WM * WN * TERMS;   // MFMAs per step
   static_assert(NS >= 3, "stages");
   static constexpr int LPS = (NLD + NM - 1) / NM;   // loads per MFMA slice of step 1
   static_assert(NR <= NM && LPS <= 2, "one read and at most two loads per MFMA slice");
@@ -123,6 +127,7 @@ struct Cfg {
   static constexpr int REGION = 32 * (32 * WN + 8) * 2, RPA = A_BYTES / REGION, RPB = B_BYTES / REGION;
   static_assert(NW <= NS * (RPA + RPB), "epilogue transpose regions");
   // Q8 block: two waves per SIMD (one wave's scale FMAs beside the other's MFMAs)
+  static_assert(!(QB && SA), "f32 activations take the plain or hi/lo panel");
   static_assert(!QB || (WM == 2 && WN == 2 && NW * OCC == 8), "Q8 block mode: 2 x 2-fragment waves, two per SIMD");
 };
 
@@ -152,19 +157,20 @@ __device__ __forceinline__ void wait_vm_lgkm0() {
   __builtin_amdgcn_s_waitcnt((V & 15) | ((V >> 4) << 14) | (7 << 4));
 }
 
-template <int WM, int WN, int MODE, int NW>
-__global__ __launch_bounds__(64 * NW, occupancy(WM, WN, NW)) void dense3_kernel(const uint16_t* __restrict__ ah, const uint16_t* __restrict__ bh,
+template <int WM, int WN, int MODE, int NW, bool SA>
+__global__ __launch_bounds__(64 * NW, occupancy(WM, WN, NW, SA)) void dense3_kernel(const uint16_t* __restrict__ ah, const uint16_t* __restrict__ al, const uint16_t* __restrict__ bh,
                                                       const uint16_t* __restrict__ bl, const float* __restrict__ dsc,
                                                       const float* __restrict__ inv,
                                                       uint32_t M, uint32_t N, uint32_t kp, void* __restrict__ y,
                                                       uint32_t y_bf16, float* __restrict__ partial,
                                                       uint32_t kt_per_split, uint32_t tiles_m,
                                                       const int32_t* __restrict__ xe) {
-  using C = Cfg<WM, WN, MODE, NW>;
+  using C = Cfg<WM, WN, MODE, NW, SA>;
   constexpr int BM = C::BM, BN = C::BN, NS = C::NS;
   constexpr bool LO = C::LO, QB = C::QB;
 #define VXT_STAGE(k)                                                                  \
   __shared__ __attribute__((aligned(1024))) char sA##k[k < NS ? C::A_BYTES : 16];     \
+  __shared__ __attribute__((aligned(1024))) char sM##k[k < NS && SA ? C::A_BYTES : 16]; \
   __shared__ __attribute__((aligned(1024))) char sB##k[k < NS ? C::B_BYTES : 16];     \
   __shared__ __attribute__((aligned(1024))) char sL##k[k < NS && LO ? C::B_BYTES : 16]; \
   __shared__ __attribute__((aligned(256))) char sD##k[k < NS ? C::D_BYTES : 16];
@@ -179,6 +185,11 @@ __global__ __launch_bounds__(64 * NW, occupancy(WM, WN, NW)) void dense3_kernel(
     constexpr int k = decltype(k_)::value;
     if constexpr (k == 0) return sA0; else if constexpr (k == 1) return sA1; else if constexpr (k == 2) return sA2;
     else if constexpr (k == 3) return sA3; else return sA4;
+  };
+  auto stM = [&](auto k_) -> char* {
+    constexpr int k = decltype(k_)::value;
+    if constexpr (k == 0) return sM0; else if constexpr (k == 1) return sM1; else if constexpr (k == 2) return sM2;
+    else if constexpr (k == 3) return sM3; else return sM4;
   };
   auto stB = [&](auto k_) -> char* {
     constexpr int k = decltype(k_)::value;
@@ -220,6 +231,7 @@ __global__ __launch_bounds__(64 * NW, occupancy(WM, WN, NW)) void dense3_kernel(
 
   const size_t pa = (size_t)((M + 15u) & ~15u) * kp * 2, pb = (size_t)((N + 15u) & ~15u) * kp * 2;   // padded planes
   const __amdgpu_buffer_rsrc_t ra = rsrc(ah, pa);
+  const __amdgpu_buffer_rsrc_t ras = rsrc(SA ? al : ah, pa);
   const __amdgpu_buffer_rsrc_t rb = rsrc(bh, pb);
   const __amdgpu_buffer_rsrc_t rl = rsrc(LO ? bl : bh, pb);
   const uint32_t nblk = kp / BK;   // Q8 block scales per weight row
@@ -238,7 +250,7 @@ __global__ __launch_bounds__(64 * NW, occupancy(WM, WN, NW)) void dense3_kernel(
 #pragma unroll
     for (int j = 0; j < C::NB; ++j) vb[j] = off(std::min(n0 + 16 * (wave + NW * j) + r16, N - 1));
   }
-  // Load piece j (A pieces, then W, then W's lo plane) of slice tile t into
+  // Load piece j (A pieces, their lo plane, then W, then W's lo plane) of slice tile t into
   // stage k.
   auto load_piece = [&](auto k_, int j, uint32_t t) {
     const uint32_t so = t * 1024u;   // the next piece of the same 16 rows
@@ -246,11 +258,14 @@ __global__ __launch_bounds__(64 * NW, occupancy(WM, WN, NW)) void dense3_kernel(
       dma4(rd, stD(k_) + 256 * (wave & 1), vd, t * 4);
     } else if (j < C::NA) {
       dma16(ra, stA(k_) + 1024 * (wave + NW * j), va[j], so);
-    } else if (j < C::NA + C::NB) {
+    } else if (j < C::NA + C::NS_A) {
       const int q = j - C::NA;
+      dma16(ras, stM(k_) + 1024 * (wave + NW * q), va[q], so);
+    } else if (j < C::NA + C::NS_A + C::NB) {
+      const int q = j - C::NA - C::NS_A;
       dma16(rb, stB(k_) + 1024 * (wave + NW * q), vb[q], so);
     } else {
-      const int q = j - C::NA - C::NB;
+      const int q = j - C::NA - C::NS_A - C::NB;
       dma16(rl, stL(k_) + 1024 * (wave + NW * q), vb[q], so);
     }
   };
@@ -258,7 +273,8 @@ __global__ __launch_bounds__(64 * NW, occupancy(WM, WN, NW)) void dense3_kernel(
   if (tid < BM) s_xe[tid] = xe[std::min(m0 + tid, M - 1)];
 
   float16v acc[WM][WN];
-  float16v accl[LO ? WM : 1][LO ? WN : 1];
+  constexpr bool SUM2 = LO || SA;   // a second accumulator of the terms times 2^-11
+  float16v accl[SUM2 ? WM : 1][SUM2 ? WN : 1];
   // Q8 block mode: the block's fragments, and the scales of this lane's
   // output columns for the tile being multiplied (set t & 1) and the one
   // being scaled
@@ -281,7 +297,7 @@ __global__ __launch_bounds__(64 * NW, occupancy(WM, WN, NW)) void dense3_kernel(
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         acc[i][j][r] = 0.0f;
-        if constexpr (LO) accl[i][j][r] = 0.0f;
+        if constexpr (SUM2) accl[i][j][r] = 0.0f;
       }
 
   // fragment (i, step s): operand rows base + 32 i + l32, logical chunk 2 s + h
@@ -293,31 +309,34 @@ __global__ __launch_bounds__(64 * NW, occupancy(WM, WN, NW)) void dense3_kernel(
     offB[s] = (wn * (32 * WN) + l32) * 64 + pos;
   }
 
-  half8 af[2][WM], bf[2][WN], lf[2][LO ? WN : 1];
+  half8 af[2][WM], mf[2][SA ? WM : 1], bf[2][WN], lf[2][LO ? WN : 1];
   // fragment read q of step s from stage k into register set `set`, in the
-  // order the step's MFMAs need them: A0, B0 .. B(WN-1) (each with its lo
-  // plane), A1 .. A(WM-1)
+  // order the step's MFMAs need them: A0, B0 .. B(WN-1), A1 .. A(WM-1), each
+  // with its lo plane
   auto read = [&](auto k_, auto s_, auto set_, auto q_) {
     constexpr int s = decltype(s_)::value, set = decltype(set_)::value, q = decltype(q_)::value;
-    constexpr int NBL = WN * (LO ? 2 : 1);
-    if constexpr (q == 0) {
-      af[set][0] = *reinterpret_cast<const half8*>(stA(k_) + offA[s]);
-    } else if constexpr (q <= NBL) {
-      constexpr int j = (q - 1) / (LO ? 2 : 1);
-      if constexpr (LO && (q - 1) % 2 == 1)
+    constexpr int NBL = WN * (LO ? 2 : 1), NA1 = SA ? 2 : 1;
+    if constexpr (q >= NA1 && q < NA1 + NBL) {
+      constexpr int j = (q - NA1) / (LO ? 2 : 1);
+      if constexpr (LO && (q - NA1) % 2 == 1)
         lf[set][j] = *reinterpret_cast<const half8*>(stL(k_) + j * 2048 + offB[s]);
       else
         bf[set][j] = *reinterpret_cast<const half8*>(stB(k_) + j * 2048 + offB[s]);
     } else {
-      constexpr int i = q - NBL;
-      af[set][i] = *reinterpret_cast<const half8*>(stA(k_) + i * 2048 + offA[s]);
+      constexpr int e = q < NA1 ? q : q - NBL, i = e / NA1;
+      if constexpr (SA && e % 2 == 1)
+        mf[set][i] = *reinterpret_cast<const half8*>(stM(k_) + i * 2048 + offA[s]);
+      else
+        af[set][i] = *reinterpret_cast<const half8*>(stA(k_) + i * 2048 + offA[s]);
     }
   };
   auto mma = [&](auto set_, auto q_) {
     constexpr int set = decltype(set_)::value, q = decltype(q_)::value;
-    constexpr int p = LO ? q / 2 : q;
+    constexpr int p = q / C::TERMS, term = q % C::TERMS;   // terms: hi hi, then (LO) hi lo, then (SA) lo hi
     constexpr int i = p / WN, j = p % WN;
-    if constexpr (LO && q % 2 == 1)
+    if constexpr (SA && term == C::TERMS - 1)
+      accl[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(mf[set][i], bf[set][j], accl[i][j], 0, 0, 0);
+    else if constexpr (LO && term == 1)
       accl[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[set][i], lf[set][j], accl[i][j], 0, 0, 0);
     else if constexpr (QB)   // step 0 (set 0) starts the block's fragment
       tmp[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[set][i], bf[set][j], set == 0 ? float16v{} : tmp[i][j],
@@ -405,7 +424,7 @@ __global__ __launch_bounds__(64 * NW, occupancy(WM, WN, NW)) void dense3_kernel(
   const bool to_partial = gridDim.y > 1;
   auto value = [&](int i, int j, int r) {
     float v = acc[i][j][r];
-    if constexpr (LO) v = hilo_combine(v, accl[i][j][r]);
+    if constexpr (SUM2) v = hilo_combine(v, accl[i][j][r]);
     return v;
   };
   auto row_of = [&](int i, int r) { return (uint32_t)(wm * 32 * WM + i * 32 + h * 4 + 8 * (r >> 2) + (r & 3)); };
@@ -468,16 +487,36 @@ __global__ __launch_bounds__(64 * NW, occupancy(WM, WN, NW)) void dense3_kernel(
       }
     }
   } else if (to_partial) {
-    const bool full = m0 + BM <= M && n0 + BN <= N;
+    if (m0 + BM <= M && n0 + BN <= N) {
 #pragma unroll
-    for (int j = 0; j < WN; ++j) {
-      const uint32_t n = n0 + wn * 32 * WN + j * 32 + l32;
-      float* const pp = partial + ((size_t)blockIdx.y * M + m0) * N + n;
+      for (int j = 0; j < WN; ++j) {
+        float* const pp = partial + ((size_t)blockIdx.y * M + m0) * N + n0 + wn * 32 * WN + j * 32 + l32;
 #pragma unroll
-      for (int i = 0; i < WM; ++i)
+        for (int i = 0; i < WM; ++i)
 #pragma unroll
-        for (int r = 0; r < 16; ++r)
-          if (full || (m0 + row_of(i, r) < M && n < N)) pp[(size_t)row_of(i, r) * N] = value(i, j, r);
+          for (int r = 0; r < 16; ++r) pp[(size_t)row_of(i, r) * N] = value(i, j, r);
+      }
+    } else if (rows_fit(BM, N)) {   // ragged
+      const auto rs = rows_rsrc(partial + ((size_t)blockIdx.y * M + m0) * N, std::min(M - m0, (uint32_t)BM), N);
+#pragma unroll
+      for (int j = 0; j < WN; ++j) {
+        const uint32_t n = n0 + wn * 32 * WN + j * 32 + l32, c0 = n < N ? n * 4u : kDropped;
+#pragma unroll
+        for (int i = 0; i < WM; ++i)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) rows_store(rs, c0 + row_of(i, r) * N * 4u, value(i, j, r));
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < WN; ++j)
+#pragma unroll
+        for (int i = 0; i < WM; ++i)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const uint32_t n = n0 + wn * 32 * WN + j * 32 + l32;
+            if (m0 + row_of(i, r) < M && n < N)
+              partial[((size_t)blockIdx.y * M + m0 + row_of(i, r)) * N + n] = value(i, j, r);
+          }
     }
   } else {
 #pragma unroll
@@ -500,42 +539,49 @@ __global__ __launch_bounds__(64 * NW, occupancy(WM, WN, NW)) void dense3_kernel(
   }
 }
 
-template <int WM, int WN, int MODE, int NW = 4>
-hipError_t launch(const uint16_t* ah, const uint16_t* bh, const uint16_t* bl, const float* dsc, const float* inv, uint32_t m,
-                  uint32_t n, uint32_t kp, void* y, bool y_bf16, float* partial, uint32_t splits,
-                  uint32_t kt_per_split, const int32_t* xe, hipStream_t s) {
-  using C = Cfg<WM, WN, MODE, NW>;
-  const uint32_t tiles_m = (m + C::BM - 1) / C::BM;
-  hipLaunchKernelGGL((dense3_kernel<WM, WN, MODE, NW>), dim3(tiles_m * ((n + C::BN - 1) / C::BN), splits), dim3(C::NT), 0,
-                     s, ah, bh, bl, dsc, inv, m, n, kp, y, (uint32_t)y_bf16, partial, kt_per_split, tiles_m, xe);
+template <int WM, int WN, int MODE, int NW, bool SA = false>
+hipError_t launch(const D3Args& a, hipStream_t s) {
+  using C = Cfg<WM, WN, MODE, NW, SA>;
+  const uint32_t tiles_m = (a.m + C::BM - 1) / C::BM;
+  hipLaunchKernelGGL((dense3_kernel<WM, WN, MODE, NW, SA>), dim3(tiles_m * ((a.n + C::BN - 1) / C::BN), a.splits),
+                     dim3(C::NT), 0, s, a.ah, a.al, a.bh, a.bl, a.dsc, a.inv, a.m, a.n, a.kp, a.y, (uint32_t)a.y_bf16,
+                     a.partial, a.kt_per_split, tiles_m, a.xe);
   return hipGetLastError();
 }
 
 }  // namespace g3
 
 // Large-tile dense phase.  cfg selects the wave tile (WM x WN fragments) and
-// the waves per workgroup: 0 = 4 x 4, 4 waves (workgroup tile 256 x 256),
-// 1 = 4 x 3, 4 waves (256 x 192), 2 = 4 x 2, 4 waves (256 x 128), 3 = 2 x 2,
-// 4 waves (128 x 128), 4 = 2 x 2, 8 waves (256 x 128).  wmode 0 = plain f16
-// panel (cfg 0-3), 1 = hi/lo panel (bh + bl * 2^-11; cfg 3 and 4), 2 = Q8
-// block (int8 values as f16 in bh, f32 scales dsc [n][kp / 32]; cfg 3 and 4).  ah, bh and bl are planes of 1 KB
-// pieces (16 rows x 32 columns, rows padded to 16).  kt_per_split counts
-// 32-column K tiles; kp % 32 == 0.
-hipError_t launch_dense3(int cfg, int wmode, const uint16_t* ah, const uint16_t* bh, const uint16_t* bl,
-                         const float* dsc, const float* inv, uint32_t m, uint32_t n, uint32_t kp, void* y, bool y_bf16,
-                         float* partial, uint32_t splits, uint32_t kt_per_split, const int32_t* xe, hipStream_t s) {
-  if (kp % g3::BK != 0 || xe == nullptr || m == 0 || n == 0 || kt_per_split == 0) return hipErrorInvalidValue;
-#define VXT_D3(WM, WN, MODE, NW) \
-  return g3::launch<WM, WN, MODE, NW>(ah, bh, bl, dsc, inv, m, n, kp, y, y_bf16, partial, splits, kt_per_split, xe, s)
+// the waves per workgroup: 1 = 4 x 3, 4 waves (workgroup tile 256 x 192), 2 =
+// 4 x 2, 4 waves (256 x 128), 3 = 2 x 2, 4 waves (128 x 128), 4 = 2 x 2, 8
+// waves (256 x 128).  wmode 0 = plain f16 panel (cfg 1-3), 1 = hi/lo panel (bh +
+// bl * 2^-11; cfg 3 and 4), 2 = Q8 block (int8 values as f16 in bh, f32 scales
+// dsc [n][kp / 32]; cfg 3 and 4).  With al, the activations' lo plane (f32 x),
+// cfg 3 and 4 of modes 0 and 1.
+// ah, al, bh and bl are planes of 1 KB pieces (16 rows x 32 columns, rows
+// padded to 16).  kt_per_split counts 32-column K tiles; kp % 32 == 0.
+hipError_t launch_dense3(int cfg, int wmode, const D3Args& a, hipStream_t s) {
+  if (a.kp % g3::BK != 0 || a.xe == nullptr || a.m == 0 || a.n == 0 || a.kt_per_split == 0) return hipErrorInvalidValue;
+  if (a.al) {
+    switch (wmode * 16 + cfg) {
+      case g3::kPlain * 16 + 3: return g3::launch<2, 2, g3::kPlain, 4, true>(a, s);
+      case g3::kPlain * 16 + 4: return g3::launch<2, 2, g3::kPlain, 8, true>(a, s);
+      case g3::kHiLo * 16 + 3: return g3::launch<2, 2, g3::kHiLo, 4, true>(a, s);
+      case g3::kHiLo * 16 + 4: return g3::launch<2, 2, g3::kHiLo, 8, true>(a, s);
+      default: return hipErrorInvalidValue;
+    }
+  }
+#define VXT_D3(WM, WN, MODE, NW)                                                 \
+  case MODE * 16 + (WM == 2 ? (NW == 4 ? 3 : 4) : WN == 3 ? 1 : 2):             \
+    return g3::launch<WM, WN, MODE, NW>(a, s);
   switch (wmode * 16 + cfg) {
-    case g3::kPlain * 16 + 0: VXT_D3(4, 4, g3::kPlain, 4);
-    case g3::kPlain * 16 + 1: VXT_D3(4, 3, g3::kPlain, 4);
-    case g3::kPlain * 16 + 2: VXT_D3(4, 2, g3::kPlain, 4);
-    case g3::kPlain * 16 + 3: VXT_D3(2, 2, g3::kPlain, 4);
-    case g3::kHiLo * 16 + 3: VXT_D3(2, 2, g3::kHiLo, 4);
-    case g3::kHiLo * 16 + 4: VXT_D3(2, 2, g3::kHiLo, 8);
-    case g3::kQBlock * 16 + 3: VXT_D3(2, 2, g3::kQBlock, 4);
-    case g3::kQBlock * 16 + 4: VXT_D3(2, 2, g3::kQBlock, 8);
+    VXT_D3(4, 3, g3::kPlain, 4)
+    VXT_D3(4, 2, g3::kPlain, 4)
+    VXT_D3(2, 2, g3::kPlain, 4)
+    VXT_D3(2, 2, g3::kHiLo, 4)
+    VXT_D3(2, 2, g3::kHiLo, 8)
+    VXT_D3(2, 2, g3::kQBlock, 4)
+    VXT_D3(2, 2, g3::kQBlock, 8)
     default: return hipErrorInvalidValue;
   }
 #undef VXT_D3

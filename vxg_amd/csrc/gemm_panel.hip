@@ -54,9 +54,7 @@ hipError_t blas_gemm_f16_tn(const uint16_t* A, uint32_t lda, const uint16_t* B, 
 hipError_t launch_dense2(int wmode, const uint16_t* ah, const uint16_t* bh, const uint16_t* bl, const float* dsc,
                          const float* inv, uint32_t m, uint32_t n, uint32_t kp, void* y, bool y_bf16, float* partial,
                          uint32_t splits, uint32_t kt_per_split, const int32_t* xe, hipStream_t s);
-hipError_t launch_dense3(int cfg, int wmode, const uint16_t* ah, const uint16_t* bh, const uint16_t* bl,
-                         const float* dsc, const float* inv, uint32_t m, uint32_t n, uint32_t kp, void* y, bool y_bf16,
-                         float* partial, uint32_t splits, uint32_t kt_per_split, const int32_t* xe, hipStream_t s);
+hipError_t launch_dense3(int cfg, int wmode, const D3Args& a, hipStream_t s);
 
 namespace gp {
 
@@ -818,6 +816,9 @@ __global__ __launch_bounds__(THREADS) void reduce_kernel(const float* __restrict
 
 // ---- planning ------------------------------------------------------------------
 
+// The per-row activation exponents at the head of the workspace.
+inline size_t xe_bytes(uint32_t m) { return al256((size_t)m * 4); }
+
 struct Plan {
   int bm, bn, wmode;
   bool lib;   // dense phase on the vendor library (gemm_blas.cpp)
@@ -876,6 +877,7 @@ inline Plan plan(const DevTensor& t, uint32_t m, bool x_bf16, bool lib) {
   // (258 / 221 vs 259 / 227 in four).
   pl.d3cfg = -1;
   pl.d3mode = 0;
+  Plan staged = pl;   // on the register-staged kernels
   const uint32_t t128 = ((m + 127) / 128) * ((t.rows + 127) / 128);
   // The large-tile kernel reads each plane through a buffer resource of at
   // most 2^31 - 16 bytes (and 32-bit lane offsets): larger planes take
@@ -883,7 +885,25 @@ inline Plan plan(const DevTensor& t, uint32_t m, bool x_bf16, bool lib) {
   const size_t kRsrcMax = 0x7ffffff0u;
   const bool fits = (size_t)((m + 15u) & ~15u) * pl.kp * 2 <= kRsrcMax &&
                     (size_t)((t.rows + 15u) & ~15u) * pl.kp * 2 <= kRsrcMax;
-  if (x_bf16 && !lib && t128 >= 96 && fits) {
+  // f32 activations (a hi and a lo plane, one more MFMA per product): in at
+  // least the K ranges of the register-staged kernel, more up to about one
+  // workgroup per CU while a range keeps 8 K tiles; 256 x 128 tiles of 8 waves
+  // where these and their ranges fill the chip, else 128 x 128.  Whole call, us,
+  // cb4 / g64 / Q8, against the register-staged kernel: 500 tokens 2048 -> 2048
+  // 35.6 / 30.2 / 33.8 (41.0 / 33.3 / 39.0); 300, 2048 -> 6144 60.4 / 42.8 / 55.6
+  // (90.3 / 67.5 / 86.8; 64.5 / 44.5 / 60.1 on 128 x 128); 2048, 2048 -> 2048 71.3 /
+  // 55.7 / 67.9 (96.0 / 76.8 / 92.8).  Up to 128 tokens, and below 32 tiles (64 up to
+  // 191 tokens), the other's 64-row tiles fill more of the chip.
+  if (!x_bf16 && !lib && m > 128 && t128 >= (m >= 192 ? 32u : 64u) && fits) {
+    pl.d3mode = pl.wmode == kWPlain ? 0 : 1;
+    pl.d3cfg = ((m + 255) / 256) * ((t.rows + 127) / 128) * pl.splits >= 192 ? 4 : 3;
+  }
+  // bf16 below 96 tiles: up to 255 tokens the register-staged kernel has 64 x 64
+  // tiles, which read each operand twice as often; this one is ahead from 48 tiles,
+  // with K >= 4096 from 32 (Q4_0, whole call: 72 tokens 2048 -> 6144 34.8 -> 31.6 us,
+  // 200 36.3 -> 29.9, 70 of 4096 -> 8192 49.4 -> 43.5).
+  const bool few = t128 < 96;
+  if (x_bf16 && !lib && fits && (!few || (m < 256 && (t128 >= 48 || (t128 >= 32 && ktiles >= 64))))) {
     pl.d3mode = pl.wmode == kWPlain ? 0 : pl.wmode == kWHiLo ? 1 : 2;
     const uint32_t m256 = (m + 255) / 256, t256 = m256 * ((t.rows + 127) / 128);
     if (pl.wmode == kWPlain && t.rows % 192 == 0 && m256 * (t.rows / 192) >= 192)
@@ -900,23 +920,42 @@ inline Plan plan(const DevTensor& t, uint32_t m, bool x_bf16, bool lib) {
     const uint32_t tiles3 = ((m + bm - 1) / bm) * ((t.rows + bn - 1) / bn);
     const uint32_t kt32 = pl.kp / 32;
     uint32_t sp = 1;
-    if (pl.d3cfg == 3)
+    if (!x_bf16 || few) {
+      if (!x_bf16) sp = pl.splits;   // no longer sums than on the register-staged kernel
+      while (tiles3 * sp < 192 && kt32 / (sp * 2) >= 8) sp *= 2;
+    } else if (pl.d3cfg == 3) {
       sp = tiles3 < 192 && kt32 >= 16 ? 2 : 1;
-    else
+    } else {
       while (tiles3 * sp * 2 <= 256 && kt32 / (sp * 2) >= 8) sp *= 2;
+    }
     pl.kt_per_split = (kt32 + sp - 1) / sp;
     pl.splits = (kt32 + pl.kt_per_split - 1) / pl.kt_per_split;
   }
   // The large-tile kernel reads both planes in 1 KB pieces (plane_off):
   // rows rounded up to 16.
-  const bool tiled = pl.d3cfg >= 0;
-  const size_t prow = tiled ? (t.rows + 15u) & ~15u : t.rows, arow = tiled ? (m + 15u) & ~15u : m;
-  pl.panel_plane = al256(prow * pl.kp * 2);
-  pl.dsc_bytes = pl.wmode == kWQBlock ? al256((size_t)t.rows * (pl.kp / 32) * 4) : 0;
-  pl.panel_bytes = pl.panel_plane * (pl.wmode == kWHiLo ? 2 : 1) + pl.dsc_bytes + al256((size_t)t.rows * 4);
-  pl.a_plane = al256(arow * pl.kp * 2);
-  pl.a_bytes = pl.a_plane * (x_bf16 ? 1 : 2);
-  pl.partial_bytes = pl.splits > 1 ? al256((size_t)pl.splits * m * t.rows * 4) : 0;
+  auto sizes = [&](Plan& q) {
+    const bool tiled = q.d3cfg >= 0;
+    const size_t prow = tiled ? (t.rows + 15u) & ~15u : t.rows, arow = tiled ? (m + 15u) & ~15u : m;
+    q.panel_plane = al256(prow * q.kp * 2);
+    q.dsc_bytes = q.wmode == kWQBlock ? al256((size_t)t.rows * (q.kp / 32) * 4) : 0;
+    q.panel_bytes = q.panel_plane * (q.wmode == kWHiLo ? 2 : 1) + q.dsc_bytes + al256((size_t)t.rows * 4);
+    q.a_plane = al256(arow * q.kp * 2);
+    q.a_bytes = q.a_plane * (x_bf16 ? 1 : 2);
+    q.partial_bytes = q.splits > 1 ? al256((size_t)q.splits * m * t.rows * 4) : 0;
+    return q.panel_bytes + q.a_bytes + q.partial_bytes;
+  };
+  if ((!x_bf16 || few) && pl.d3cfg >= 0) {
+    // The workspace of the register-staged kernel stays the call's at the
+    // least, and a call that fits the allocation-free entry point's scratch
+    // with that kernel keeps it where only that fits.
+    const size_t before = sizes(staged), now = sizes(pl);
+    if (before + xe_bytes(m) <= kNoAllocScratch && now + xe_bytes(m) > kNoAllocScratch)
+      pl = staged;
+    else if (now < before)
+      pl.partial_bytes += before - now;
+  } else {
+    (void)sizes(pl);
+  }
   // Library: for products of fewer than 128 output tiles of 128 x 128, K
   // slices until ~256 tiles are in flight, each slice at least 1024 columns
   // and a whole number of K tiles (at 512 x 6144 outputs, 192 tiles, two
@@ -1034,8 +1073,23 @@ hipError_t run(const DevTensor& t, const void* x, bool x_bf16, uint32_t m, void*
     (void)hipGetLastError();   // no algorithm for this shape: the own dense kernel on the same panel
   }
   if (pl.d3cfg >= 0) {
-    e = launch_dense3(pl.d3cfg, pl.d3mode, ah, p.hi, p.lo, p.dsc, p.inv, m, t.rows, pl.kp, y, y_bf16, partial, pl.splits,
-                      pl.kt_per_split, xe, s);
+    D3Args a{};
+    a.ah = ah;
+    a.al = x_bf16 ? nullptr : al;
+    a.bh = p.hi;
+    a.bl = p.lo;
+    a.dsc = p.dsc;
+    a.inv = p.inv;
+    a.m = m;
+    a.n = t.rows;
+    a.kp = pl.kp;
+    a.y = y;
+    a.y_bf16 = y_bf16;
+    a.partial = partial;
+    a.splits = pl.splits;
+    a.kt_per_split = pl.kt_per_split;
+    a.xe = xe;
+    e = launch_dense3(pl.d3cfg, pl.d3mode, a, s);
   } else if (x_bf16 && pl.bm == 128) {
     // 128 x 128 tiles with bf16 (exact f16) activations: the interleaved
     // dense kernel (gemm_dense.hip), any weight mode
@@ -1169,7 +1223,7 @@ static bool library_path(int mode) { return mode == kGemmLibrary; }
 
 // Workspace: the per-row activation exponents first, then the path's own
 // (the tile path keeps its exponents in its own block).
-static size_t xe_bytes(uint32_t m) { return gp::al256((size_t)m * 4); }
+using gp::xe_bytes;
 
 static size_t path_workspace_bytes(Path path, const DevTensor& t, uint32_t m, bool x_bf16, int mode) {
   switch (path) {

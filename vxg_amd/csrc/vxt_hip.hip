@@ -69,7 +69,7 @@ void blas_release_device(int dev);
 // calls through that entry point never allocate.  Host code reaches it only
 // through the device address hipGetSymbolAddress returns for the current
 // device (kept per context); the name itself is a host-side stand-in.
-constexpr size_t kScratchBytes = (size_t)32 << 20;
+constexpr size_t kScratchBytes = vxt::kNoAllocScratch;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 namespace {
