@@ -1,8 +1,8 @@
-"""The large-tile dense kernel (gemm_dense3.hip) with f32 activations and below
-96 output tiles, at the edges of its ranges: tiles that end inside the batch and
-the rows, one and several K ranges, 4- and 8-wave workgroups, columns that end
-inside a K tile.  Reference: the decoded weights (bit-exact, the oracle) times
-the activations in 64 bits.
+"""The large-tile dense kernel (gemm_dense3.hip) with f32 activations, below 96
+output tiles and with the gated epilogue, at the edges of its ranges: tiles that
+end inside the batch and the rows, one and several K ranges, 4- and 8-wave
+workgroups, columns that end inside a K tile.  Reference: the decoded weights
+(bit-exact, the oracle) times the activations in 64 bits.
 
 Bound: an f32 operand is split as hi + lo * 2^-11 in f16 (relative error at
 most 2^-22, or 2^-36 of the row's largest entry for small ones) and the lo lo
@@ -54,4 +54,46 @@ def test_large_tile_edges(eng, kind, rows, cols, M, f32):
     W = oracle.decode_rows(m).astype(np.float64)
     err, bound = np.abs(got - Xq @ W.T), bound_of(Xq, W, cols)
     assert np.all(err <= bound), float((err / bound).max())
+    t.free()
+
+
+# Gated [gate; up] calls in one K range: batch and outputs that end inside a
+# tile, output counts that are and are not multiples of 8 pieces, 4- and 8-wave
+# workgroups and 256 x 192 tiles.  Bound: an output is act(g) u with g and u
+# within B of the exact sums; |act'| <= 1.13 and |act(g)| <= |g| for both
+# activations; 2^-18 of the result and 2^-20 |g u| for expf, tanh and
+# 1 + tanh of a negative g.  bf16 outputs are the f32 outputs' rounding.
+@pytest.mark.parametrize("n_ff,cols,M", [(6144, 520, 256), (6160, 200, 257), (9216, 320, 1050), (3072, 1030, 1000),
+                                         (2064, 640, 1999)])
+@pytest.mark.parametrize("kind", ["cb4", "g64", "q8", "q4_0"])
+def test_gated_epilogue_edges(eng, kind, n_ff, cols, M):
+    print(f"gated {kind} n_ff={n_ff} cols={cols} M={M}", flush=True)
+    seed = n_ff + M
+    m = synth.make_q40(2 * n_ff, cols, seed=seed) if kind == "q4_0" else make(kind, 2 * n_ff, cols, seed=seed)
+    t = eng.upload_packed(m)
+    xh = f32_to_bf16_bits(np.random.default_rng(seed).standard_normal((M, cols)).astype(np.float32))
+    xd = eng.to_device(xh)
+    sel = np.unique(np.r_[0:2, 31:34, M // 2, M - 18:M])
+    X = bf16_bits_to_f32(xh).reshape(M, cols)[sel].astype(np.float64)
+    W = oracle.decode_rows(m).astype(np.float64)
+    z, B = X @ W.T, bound_of(X, W, cols)
+    g, u, Bg, Bu = z[:, :n_ff], z[:, n_ff:], B[:, :n_ff], B[:, n_ff:]
+    for activation in (engine.ACT_SILU, engine.ACT_GELU_TANH):
+        out = {}
+        for dt, np_dt, sz in ((engine.DTYPE_F32, np.float32, 4), (engine.DTYPE_BF16, np.uint16, 2)):
+            ad = eng.alloc(M * n_ff * sz)
+            eng.ffn_glu_dev(t, xd.ptr, engine.DTYPE_BF16, M, ad.ptr, dt, n_ff, activation, eng.stream)
+            eng.synchronize()
+            out[dt] = ad.download(np_dt, (M, n_ff))
+            ad.free()
+        if activation == engine.ACT_SILU:
+            want = g / (1 + np.exp(-g)) * u
+        else:
+            want = 0.5 * g * (1 + np.tanh(0.7978846 * (g + 0.044715 * g ** 3))) * u
+        bound = (1.13 * (np.abs(u) + Bu) * Bg + np.abs(g) * Bu + 2.0 ** -18 * np.abs(want) +
+                 2.0 ** -20 * np.abs(g * u) + 1e-30)
+        err = np.abs(out[engine.DTYPE_F32][sel] - want)
+        assert np.all(err <= bound), (activation, float((err / bound).max()))
+        assert np.array_equal(out[engine.DTYPE_BF16].ravel(), f32_to_bf16_bits(out[engine.DTYPE_F32]).ravel())
+    xd.free()
     t.free()

@@ -169,6 +169,7 @@ struct D3Args {
   float* partial;
   uint32_t splits, kt_per_split;
   const int32_t* xe;
+  bool glu, gelu;
 };
 
 // One layer's Q8_0 KV cache (the planes of VxtKvQ8Cache): row t holds

@@ -66,6 +66,7 @@
 #include <type_traits>
 #include <utility>
 
+#include "act.hpp"
 #include "common.hpp"
 
 #pragma clang fp contract(off)
@@ -157,14 +158,14 @@ __device__ __forceinline__ void wait_vm_lgkm0() {
   __builtin_amdgcn_s_waitcnt((V & 15) | ((V >> 4) << 14) | (7 << 4));
 }
 
-template <int WM, int WN, int MODE, int NW, bool SA>
+template <int WM, int WN, int MODE, int NW, bool SA, bool GLU>
 __global__ __launch_bounds__(64 * NW, occupancy(WM, WN, NW, SA)) void dense3_kernel(const uint16_t* __restrict__ ah, const uint16_t* __restrict__ al, const uint16_t* __restrict__ bh,
                                                       const uint16_t* __restrict__ bl, const float* __restrict__ dsc,
                                                       const float* __restrict__ inv,
                                                       uint32_t M, uint32_t N, uint32_t kp, void* __restrict__ y,
                                                       uint32_t y_bf16, float* __restrict__ partial,
                                                       uint32_t kt_per_split, uint32_t tiles_m,
-                                                      const int32_t* __restrict__ xe) {
+                                                      const int32_t* __restrict__ xe, uint32_t gelu) {
   using C = Cfg<WM, WN, MODE, NW, SA>;
   constexpr int BM = C::BM, BN = C::BN, NS = C::NS;
   constexpr bool LO = C::LO, QB = C::QB;
@@ -428,6 +429,71 @@ __global__ __launch_bounds__(64 * NW, occupancy(WM, WN, NW, SA)) void dense3_ker
     return v;
   };
   auto row_of = [&](int i, int r) { return (uint32_t)(wm * 32 * WM + i * 32 + h * 4 + 8 * (r >> 2) + (r & 3)); };
+  if constexpr (GLU) {
+    // Gated [gate; up] output: the panel interleaves 16 gate rows and the 16
+    // up rows of the same outputs, so a fragment's columns 0-15 are gates and
+    // 16-31 their ups.  Exchanging a pair of rows r, r + 1 between the two
+    // 16-lane halves (v_permlane16_swap) leaves each lane one whole output:
+    // row r in the gate lanes, row r + 1 in the up lanes.
+    constexpr uint32_t LDO = 16 * WN + 8;   // elements per LDS row of 16 WN outputs
+    const uint32_t half = l32 >> 4, oc = l32 & 15u, n_ff = N / 2, o0 = (n0 + wn * 32 * WN) / 2;
+    const bool fast = y_bf16 && n_ff % 8 == 0 && n0 + BN <= N && reinterpret_cast<uintptr_t>(y) % 16 == 0;
+    auto pick = [](uint32_t k, char* a0, char* a1, char* a2, char* a3, char* a4) {
+      return k == 0 ? a0 : k == 1 ? a1 : k == 2 ? a2 : k == 3 ? a3 : a4;
+    };
+    char* rbase;
+    if (C::RPA > 0 && wave < (uint32_t)(NS * C::RPA)) {
+      rbase = pick(wave / C::RPA, sA0, sA1, sA2, sA3, sA4) + (wave % C::RPA) * C::REGION;
+    } else {
+      const uint32_t w = wave - NS * C::RPA;
+      rbase = pick(w / C::RPB, sB0, sB1, sB2, sB3, sB4) + (w % C::RPB) * C::REGION;
+    }
+    uint16_t* reg = reinterpret_cast<uint16_t*>(rbase);
+    float sc[WN];
+#pragma unroll
+    for (int j = 0; j < WN; ++j) sc[j] = inv[std::min(n0 + wn * 32 * WN + j * 32 + l32, N - 1)];
+#pragma unroll
+    for (int i = 0; i < WM; ++i) {
+#pragma unroll
+      for (int r = 0; r < 16; r += 2) {
+        const uint32_t rl0 = wm * 32 * WM + i * 32 + h * 4 + 8 * (r >> 2) + (r & 3);
+        const int e0 = -s_xe[rl0], e1 = -s_xe[rl0 + 1];
+        const uint32_t rr = h * 4 + 8 * (r >> 2) + (r & 3) + half;
+        const uint32_t m = m0 + rl0 + half;
+#pragma unroll
+        for (int j = 0; j < WN; ++j) {
+          const float a = ldexpf(value(i, j, r) * sc[j], e0), b = ldexpf(value(i, j, r + 1) * sc[j], e1);
+          const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+          const float v = gated_act(__uint_as_float(sw[0]), __uint_as_float(sw[1]), gelu != 0);
+          if (fast) {
+            reg[rr * LDO + j * 16 + oc] = f32_to_bf16(v);
+          } else {
+            const uint32_t o = o0 + j * 16 + oc;
+            if (m < M && o < n_ff) {
+              if (y_bf16)
+                static_cast<uint16_t*>(y)[(size_t)m * n_ff + o] = f32_to_bf16(v);
+              else
+                static_cast<float*>(y)[(size_t)m * n_ff + o] = v;
+            }
+          }
+        }
+      }
+      if (fast) {
+        // 32 rows x 16 WN outputs: 2 WN lanes per row, 16 bytes each
+        constexpr uint32_t LPR = 2 * WN, ROWS_PER = 64 / LPR;
+#pragma unroll
+        for (uint32_t q = 0; q < (32 + ROWS_PER - 1) / ROWS_PER; ++q) {
+          const uint32_t rr = q * ROWS_PER + lane / LPR, c = lane % LPR;
+          const uint32_t m = m0 + wm * 32 * WM + i * 32 + rr;
+          if (rr < 32 && lane < ROWS_PER * LPR && m < M) {
+            const u32x4 v = *reinterpret_cast<const u32x4*>(reg + rr * LDO + c * 8);
+            *reinterpret_cast<u32x4*>(static_cast<uint16_t*>(y) + (size_t)m * n_ff + o0 + c * 8) = v;
+          }
+        }
+      }
+    }
+    return;
+  }
   const bool rows_fast = y_bf16 && !to_partial && N % 8 == 0 && n0 + BN <= N &&
                          reinterpret_cast<uintptr_t>(y) % 16 == 0;
   if (rows_fast) {
@@ -539,13 +605,13 @@ __global__ __launch_bounds__(64 * NW, occupancy(WM, WN, NW, SA)) void dense3_ker
   }
 }
 
-template <int WM, int WN, int MODE, int NW, bool SA = false>
+template <int WM, int WN, int MODE, int NW, bool SA = false, bool GLU = false>
 hipError_t launch(const D3Args& a, hipStream_t s) {
   using C = Cfg<WM, WN, MODE, NW, SA>;
   const uint32_t tiles_m = (a.m + C::BM - 1) / C::BM;
-  hipLaunchKernelGGL((dense3_kernel<WM, WN, MODE, NW, SA>), dim3(tiles_m * ((a.n + C::BN - 1) / C::BN), a.splits),
+  hipLaunchKernelGGL((dense3_kernel<WM, WN, MODE, NW, SA, GLU>), dim3(tiles_m * ((a.n + C::BN - 1) / C::BN), a.splits),
                      dim3(C::NT), 0, s, a.ah, a.al, a.bh, a.bl, a.dsc, a.inv, a.m, a.n, a.kp, a.y, (uint32_t)a.y_bf16,
-                     a.partial, a.kt_per_split, tiles_m, a.xe);
+                     a.partial, a.kt_per_split, tiles_m, a.xe, (uint32_t)a.gelu);
   return hipGetLastError();
 }
 
@@ -557,11 +623,13 @@ hipError_t launch(const D3Args& a, hipStream_t s) {
 // waves (256 x 128).  wmode 0 = plain f16 panel (cfg 1-3), 1 = hi/lo panel (bh +
 // bl * 2^-11; cfg 3 and 4), 2 = Q8 block (int8 values as f16 in bh, f32 scales
 // dsc [n][kp / 32]; cfg 3 and 4).  With al, the activations' lo plane (f32 x),
-// cfg 3 and 4 of modes 0 and 1.
+// cfg 3 and 4 of modes 0 and 1.  With glu (one K range, no al), the panel
+// interleaves gate and up rows by 16 and y is the gated activation [m][n / 2].
 // ah, al, bh and bl are planes of 1 KB pieces (16 rows x 32 columns, rows
 // padded to 16).  kt_per_split counts 32-column K tiles; kp % 32 == 0.
 hipError_t launch_dense3(int cfg, int wmode, const D3Args& a, hipStream_t s) {
   if (a.kp % g3::BK != 0 || a.xe == nullptr || a.m == 0 || a.n == 0 || a.kt_per_split == 0) return hipErrorInvalidValue;
+  if (a.glu && (a.splits != 1 || a.al)) return hipErrorInvalidValue;
   if (a.al) {
     switch (wmode * 16 + cfg) {
       case g3::kPlain * 16 + 3: return g3::launch<2, 2, g3::kPlain, 4, true>(a, s);
@@ -573,7 +641,7 @@ hipError_t launch_dense3(int cfg, int wmode, const D3Args& a, hipStream_t s) {
   }
 #define VXT_D3(WM, WN, MODE, NW)                                                 \
   case MODE * 16 + (WM == 2 ? (NW == 4 ? 3 : 4) : WN == 3 ? 1 : 2):             \
-    return g3::launch<WM, WN, MODE, NW>(a, s);
+    return a.glu ? g3::launch<WM, WN, MODE, NW, false, true>(a, s) : g3::launch<WM, WN, MODE, NW>(a, s);
   switch (wmode * 16 + cfg) {
     VXT_D3(4, 3, g3::kPlain, 4)
     VXT_D3(4, 2, g3::kPlain, 4)

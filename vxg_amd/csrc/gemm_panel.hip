@@ -80,7 +80,17 @@ struct Panel {
   float* dsc;       // [N][kp/32] block scales (Q8 block mode)
   uint32_t kp;      // K rounded up to BK
   uint32_t tiled;   // hi / lo in 1 KB pieces (plane_off), else row-major
+  // 0, or the gate rows of a [gate; up] tensor (a multiple of 16): the panel
+  // then interleaves them by 16, gate rows 16 b .. + 15 at panel rows 32 b,
+  // their up rows at 32 b + 16 (the gated epilogue of gemm_dense3.hip).
+  uint32_t n_ff;
 };
+
+__device__ __forceinline__ uint32_t panel_row(const Panel& p, uint32_t n) {
+  if (!p.n_ff) return n;
+  const uint32_t g = n < p.n_ff ? n : n - p.n_ff;
+  return (g >> 4) * 32u + (g & 15u) + (n < p.n_ff ? 0u : 16u);
+}
 
 // How a panel represents the weights.
 enum WMode : int {
@@ -390,7 +400,8 @@ __global__ __launch_bounds__(THREADS) void panel_kernel(DevTensor t, Panel p, ui
   const uint32_t c0 = seg + 8 * lane;
   uint16_t* hi = p.hi;
   uint16_t* lo = p.lo;
-  auto at = [&](uint32_t c) { return plane_off(n, c, KP, p.tiled); };   // column c of row n
+  const uint32_t pn = panel_row(p, n);
+  auto at = [&](uint32_t c) { return plane_off(pn, c, KP, p.tiled); };   // column c of row n
   float s = 1.0f;
   if constexpr (KIND == KIND_G64) {
     // KP <= kp here (kp is a multiple of 64 and at least K).  The segment's
@@ -452,7 +463,7 @@ __global__ __launch_bounds__(THREADS) void panel_kernel(DevTensor t, Panel p, ui
     if (qblock) {   // block scales as f32; blocks past the weights' own are zero
       const uint32_t b0 = seg / 32 + lane;
       if (b0 < KP / 32)
-        p.dsc[(size_t)n * (KP / 32) + b0] = b0 < kp / 32 ? f16_to_f32_exact(dp[b0]) : 0.0f;
+        p.dsc[(size_t)pn * (KP / 32) + b0] = b0 < kp / 32 ? f16_to_f32_exact(dp[b0]) : 0.0f;
     } else {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -541,7 +552,7 @@ __global__ __launch_bounds__(THREADS) void panel_kernel(DevTensor t, Panel p, ui
       }
     }
   }
-  if (lane == 0 && seg == 0) p.inv[n] = 1.0f / s;
+  if (lane == 0 && seg == 0) p.inv[pn] = 1.0f / s;
 }
 
 // ---- phase 2: dense GEMM -----------------------------------------------------
@@ -1034,10 +1045,14 @@ hipError_t library_dense(const Panel& p, const uint16_t* ah, const uint16_t* al,
   return launch_gemm_reduce(d, splits, p.inv, xe, m, n, y, y_bf16, s);
 }
 
+enum Glu : int { kNoGlu = 0, kGluSilu = 1, kGluGelu = 2 };
+
+// glu: y is the gated activation of a [gate; up] tensor (large-tile kernel, one K range).
 template <uint32_t KIND>
 hipError_t run(const DevTensor& t, const void* x, bool x_bf16, uint32_t m, void* y, bool y_bf16, void* ws,
-               size_t ws_bytes, const int32_t* xe, hipStream_t s, bool lib) {
+               size_t ws_bytes, const int32_t* xe, hipStream_t s, bool lib, Glu glu = kNoGlu) {
   const Plan pl = plan(t, m, x_bf16, lib);
+  if (glu != kNoGlu && (pl.d3cfg < 0 || pl.splits != 1)) return hipErrorInvalidValue;
   if (ws_bytes < pl.panel_bytes + pl.a_bytes + pl.partial_bytes) return hipErrorInvalidValue;
   char* base = static_cast<char*>(ws);
   const bool hilo = pl.wmode == kWHiLo;
@@ -1048,6 +1063,7 @@ hipError_t run(const DevTensor& t, const void* x, bool x_bf16, uint32_t m, void*
   p.inv = reinterpret_cast<float*>(base + pl.panel_plane * (hilo ? 2 : 1) + pl.dsc_bytes);
   p.kp = pl.kp;
   p.tiled = pl.d3cfg >= 0;
+  p.n_ff = glu != kNoGlu ? t.rows / 2 : 0;
   uint16_t* ah = reinterpret_cast<uint16_t*>(base + pl.panel_bytes);
   uint16_t* al = reinterpret_cast<uint16_t*>(base + pl.panel_bytes + (x_bf16 ? 0 : pl.a_plane));
   float* partial = reinterpret_cast<float*>(base + pl.panel_bytes + pl.a_bytes);
@@ -1089,6 +1105,8 @@ hipError_t run(const DevTensor& t, const void* x, bool x_bf16, uint32_t m, void*
     a.splits = pl.splits;
     a.kt_per_split = pl.kt_per_split;
     a.xe = xe;
+    a.glu = glu != kNoGlu;
+    a.gelu = glu == kGluGelu;
     e = launch_dense3(pl.d3cfg, pl.d3mode, a, s);
   } else if (x_bf16 && pl.bm == 128) {
     // 128 x 128 tiles with bf16 (exact f16) activations: the interleaved
@@ -1313,6 +1331,40 @@ hipError_t launch_gemm(const DevTensor& t, const void* x, bool x_bf16, uint32_t 
     case KIND_Q8: return gp::run<KIND_Q8>(t, x, x_bf16, m, y, y_bf16, rest, rest_bytes, xe, s, lib);
     case KIND_Q40: return gp::run<KIND_Q40>(t, x, x_bf16, m, y, y_bf16, rest, rest_bytes, xe, s, lib);
     case KIND_CB4: return gp::run<KIND_CB4>(t, x, x_bf16, m, y, y_bf16, rest, rest_bytes, xe, s, lib);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+// Gated prefill in one pass over the GEMM's outputs: whether a [gate; up] call
+// takes the panel and the large-tile kernel with the gated epilogue, instead of
+// f32 gate and up rows in the workspace and an element-wise pass over them.
+// From 256 tokens, where that kernel runs in one K range (2048 -> 2 x 6144, us,
+// this against the staged form: g64 1024 tokens 75.3 against 97.3; cb4 500
+// tokens 81.5 against 90.9, Q8 58.4 against 69.1, Q4_0 57.5 against 67.3).
+bool gemm_glu_takes(const DevTensor& t, uint32_t m, bool x_bf16, uint32_t act_stride, int mode) {
+  if ((mode != kGemmAuto && mode != kGemmAutoOwn) || !x_bf16 || m < 256) return false;
+  if (t.rows % 32 != 0 || act_stride != t.rows / 2) return false;
+  const gp::Plan pl = gp::plan(t, m, true, false);
+  return pl.d3cfg >= 0 && pl.splits == 1;
+}
+
+size_t gemm_glu_workspace_bytes(const DevTensor& t, uint32_t m) {
+  const gp::Plan pl = gp::plan(t, m, true, false);
+  return xe_bytes(m) + pl.panel_bytes + pl.a_bytes;
+}
+
+hipError_t launch_gemm_glu(const DevTensor& t, const void* x, uint32_t m, void* act, bool act_bf16, bool gelu, void* ws,
+                           size_t ws_bytes, hipStream_t s) {
+  if (ws_bytes < gemm_glu_workspace_bytes(t, m)) return hipErrorInvalidValue;
+  int32_t* xe = static_cast<int32_t*>(ws);
+  void* rest = static_cast<char*>(ws) + xe_bytes(m);
+  const size_t rest_bytes = ws_bytes - xe_bytes(m);
+  const gp::Glu g = gelu ? gp::kGluGelu : gp::kGluSilu;
+  switch (t.kind) {
+    case KIND_G64: return gp::run<KIND_G64>(t, x, true, m, act, act_bf16, rest, rest_bytes, xe, s, false, g);
+    case KIND_Q8: return gp::run<KIND_Q8>(t, x, true, m, act, act_bf16, rest, rest_bytes, xe, s, false, g);
+    case KIND_Q40: return gp::run<KIND_Q40>(t, x, true, m, act, act_bf16, rest, rest_bytes, xe, s, false, g);
+    case KIND_CB4: return gp::run<KIND_CB4>(t, x, true, m, act, act_bf16, rest, rest_bytes, xe, s, false, g);
     default: return hipErrorInvalidValue;
   }
 }

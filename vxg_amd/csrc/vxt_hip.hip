@@ -57,6 +57,10 @@ hipError_t launch_attn_prefill(const KvQ8Dev& c, const float* q, const float* ga
 size_t greedy_state_bytes();
 hipError_t launch_greedy(const float* logits, uint32_t n, void* state, uint32_t* out, hipStream_t s);
 hipError_t launch_read_probe(const void* p, size_t bytes, uint32_t* sink, uint32_t key, hipStream_t s);
+bool gemm_glu_takes(const DevTensor& t, uint32_t m, bool x_bf16, uint32_t act_stride, int mode);
+size_t gemm_glu_workspace_bytes(const DevTensor& t, uint32_t m);
+hipError_t launch_gemm_glu(const DevTensor& t, const void* x, uint32_t m, void* act, bool act_bf16, bool gelu, void* ws,
+                           size_t ws_bytes, hipStream_t s);
 bool skinny_glu_takes(const DevTensor& t, const void* x, uint32_t m, bool x_bf16, int mode);
 hipError_t launch_skinny_glu(const DevTensor& t, const void* x, bool x_bf16, uint32_t m, void* act, bool act_bf16,
                              uint32_t act_stride, bool gelu, hipStream_t s);
@@ -935,7 +939,7 @@ int vxt_hip_ffn_glu_dev(void* ctx, void* tensor, const void* x, uint32_t x_dtype
       e = vxt::launch_gemv_glu(d, x, xb, 1, act, ab, act_stride, gelu, s);
     } else {
       // The workspace of the staged form: the GEMM's own, then gate and up
-      // rows in f32.  The fused few-token form uses none of it; what a call
+      // rows in f32.  The fused forms use less of it or none; what a call
       // reserves does not depend on the form.
       const size_t gemm_ws =
           batch_m > 8 ? (vxt::gemm_workspace_bytes(d, batch_m, xb, c->gemm_mode) + 255) / 256 * 256 : 0;
@@ -943,6 +947,9 @@ int vxt_hip_ffn_glu_dev(void* ctx, void* tensor, const void* x, uint32_t x_dtype
       if (batch_m > 2) ensure_ws(c, gemm_ws + stage, s);
       if (vxt::skinny_glu_takes(d, x, batch_m, xb, c->gemm_mode)) {
         e = vxt::launch_skinny_glu(d, x, xb, batch_m, act, ab, act_stride, gelu, s);
+      } else if (vxt::gemm_glu_takes(d, batch_m, xb, act_stride, c->gemm_mode) &&
+                 vxt::gemm_glu_workspace_bytes(d, batch_m) <= gemm_ws + stage) {
+        e = vxt::launch_gemm_glu(d, x, batch_m, act, ab, gelu, c->ws, gemm_ws + stage, s);
       } else {
         float* gu = reinterpret_cast<float*>(static_cast<char*>(c->ws) + gemm_ws);
         e = batch_m <= 8 ? vxt::launch_gemv(d, x, xb, true, batch_m, gu, false, s)
