@@ -311,3 +311,64 @@ def test_step_errors(eng):
     finally:
         buf.free()
         cache.free()
+
+
+@pytest.mark.parametrize("pos0,m,n_head,n_kv,hd", [
+    (0, 128, 16, 16, 128), (0, 129, 4, 1, 128), (112, 16, 8, 1, 32), (127, 18, 6, 2, 64), (900, 33, 16, 2, 128),
+    (3970, 125, 4, 4, 64), (4100, 40, 8, 8, 32)])
+def test_prefill_segments_match_oracle(eng, pos0, m, n_head, n_kv, hd):
+    """Small prefill grids walk the positions in segments of 4 to 16 tiles of
+    32 (the last rows of one segment, the first of the next, the most segments
+    a token has); the bar is the oracle's as above."""
+    print(f"prefill segments pos0={pos0} m={m} heads={n_head}/{n_kv} hd={hd}", flush=True)
+    case = Case(eng, n_head, n_kv, hd, gated=True, norms=True, neox=True, rope_dim=hd, seed=pos0 + m)
+    cache = eng.kv_q8_cache(pos0 + m, n_kv, hd)
+    try:
+        if pos0:
+            run_step(eng, case, cache, *case.tokens(pos0), 0, 0)
+        q, k, v = case.tokens(m)
+        out = run_step(eng, case, cache, q, k, v, pos0, pos0)
+        qi, _, _ = case.host_inputs(q, k, v)
+        kb, vb = cache.blocks("k", pos0 + m), cache.blocks("v", pos0 + m)
+        for t in sorted({0, 1, m // 2, m - 2, m - 1}):
+            L = pos0 + t + 1
+            qh, qg = oracle_q(case, qi[t], pos0 + t)
+            ref = oracle.attn_q8(qh, kb[:L], vb[:L], L, n_head, n_kv, hd, gate=qg)
+            vmax = np.abs(oracle.q8_dequant(vb[:L].reshape(-1))).max()
+            assert np.abs(out[t] - ref).max() <= 1e-4 * vmax, t
+    finally:
+        cache.free()
+        case.free()
+
+
+def test_prefill_in_a_capture_with_little_workspace():
+    """A capture whose workspace holds the prepared queries but no segments'
+    sums still records the step: one walk per row, the eager result within
+    rounding (the two add a row's tiles in another order)."""
+    e = engine.HipEngine()
+    small, case = Case(e, 16, 16, 128, gated=True, seed=3), Case(e, 8, 8, 128, gated=True, seed=4)
+    c0, cache = e.kv_q8_cache(112, 16, 128), e.kv_q8_cache(200, 8, 128)
+    bufs = []
+    try:
+        run_step(e, small, c0, *small.tokens(112), 0, 0)      # one segment: the queries only
+        bufs = [e.to_device(np.ascontiguousarray(a, np.float32)) for a in case.tokens(200)]
+        od = e.alloc(200 * 8 * 128 * 4)
+        bufs.append(od)
+        step = lambda s: cache.step(case.params, bufs[0].ptr, bufs[1].ptr, bufs[2].ptr, 0, 0, od.ptr, batch_m=200,
+                                    q_stride=case.p.q_rows, kv_stride=case.kvd,
+                                    stream=s)
+        g = e.capture(step)
+        g.launch(1)
+        got = od.download(np.float32, (200, 8 * 128))
+        g.free()
+        step(e.stream)
+        e.synchronize()
+        want = od.download(np.float32, (200, 8 * 128))
+        vmax = np.abs(oracle.q8_dequant(cache.blocks("v", 200).reshape(-1))).max()
+        assert np.abs(got - want).max() <= 1e-4 * vmax
+    finally:
+        for b in bufs:
+            b.free()
+        for c in (c0, cache, small, case):
+            c.free()
+        e.close()

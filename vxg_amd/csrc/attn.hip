@@ -51,7 +51,7 @@ constexpr uint32_t kMaxGroup = 8;   // query heads per kv head
 typedef float float16v __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-constexpr uint32_t kSegTiles = 16;   // prefill: 32-position tiles per position segment
+constexpr uint32_t kSegTiles = 16;   // prefill: 32-position tiles per position segment, at most
 
 // f32 -> f16 bits, round to nearest even with f16 subnormals kept and
 // overflow to infinity: what fp16.rs:33-77 computes with integer steps, here
@@ -734,7 +734,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_bf16_kernel(KvQ8Dev c, co
                                                                 const float* __restrict__ gate,
                                                                 float* __restrict__ out, float* __restrict__ part,
                                                                 uint32_t n_head, uint32_t group, uint32_t tq,
-                                                                uint32_t pos0, uint32_t batch) {
+                                                                uint32_t pos0, uint32_t batch, uint32_t seg_tiles) {
   constexpr uint32_t TP = 32, NST = HD / 16, NB = HD / 32;
   constexpr uint32_t KST = HD + 8, VST = TP + 8;        // bf16 strides
   constexpr uint32_t NPC = (TP / 2) * (HD / 8);         // pieces: 2 positions x 8 dims
@@ -753,9 +753,9 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_bf16_kernel(KvQ8Dev c, co
   const uint32_t my_pos = pos0 + tkc, first_pos = pos0 + tb;
   const uint32_t head = kvh * group + g;
   const uint32_t last = pos0 + t_end - 1u;
-  const uint32_t tile0 = blockIdx.z * kSegTiles;
+  const uint32_t tile0 = blockIdx.z * seg_tiles;
   if (tile0 * TP > last) return;
-  const uint32_t n_tiles = gridDim.z == 1 ? last / TP + 1u : min(last / TP + 1u, tile0 + kSegTiles);
+  const uint32_t n_tiles = gridDim.z == 1 ? last / TP + 1u : min(last / TP + 1u, tile0 + seg_tiles);
   const uint32_t row_q = c.n_kv * HD, row_d = c.n_kv * (HD / 32);
   const float scale2 = 1.4426950408889634f / sqrtf((float)HD);
 
@@ -1122,41 +1122,73 @@ hipError_t launch_attn(const KvQ8Dev& c, const float* q, uint32_t n_head, uint32
 // Causal attention of batch prepared queries (q, gate: [batch][n_head][hd])
 // on MFMA: tokens at positions pos0 .. pos0 + batch - 1, every cache row up to
 // the last written.  hd <= 128.  Positions are cut into segments of
-// kSegTiles * 32 when there are more than one; ws then holds
-// attn_prefill_workspace_bytes(...) of partial sums.
-uint32_t prefill_segments(uint32_t pos0, uint32_t batch) {
-  return (pos0 + batch - 1u) / (kSegTiles * 32u) + 1u;
+// seg_tiles * 32 when there are more than one; ws then holds
+// prefill_part_bytes(...) of partial sums.
+uint32_t prefill_segments(uint32_t pos0, uint32_t batch, uint32_t seg_tiles) {
+  return (pos0 + batch - 1u) / (seg_tiles * 32u) + 1u;
 }
 
-size_t attn_prefill_workspace_bytes(uint32_t n_head, uint32_t hd, uint32_t pos0, uint32_t batch) {
-  const uint32_t ns = prefill_segments(pos0, batch);
+size_t prefill_part_bytes(uint32_t n_head, uint32_t hd, uint32_t pos0, uint32_t batch, uint32_t seg_tiles) {
+  const uint32_t ns = prefill_segments(pos0, batch, seg_tiles);
   return ns > 1 ? (size_t)batch * n_head * ns * (hd + 2) * sizeof(float) : 0;
 }
 
+// The segment length: kSegTiles, halved down to 4 tiles while the grid stays
+// within the 512 workgroups that run at once, a token has at most 32 segments
+// and the partial sums fit ws_bytes.  A workgroup walks its tiles one after the
+// other, about 3 us each, and a short prompt has few of them: 500 tokens, 16
+// heads x 128, are 64 workgroups of up to 16 tiles, 52 us; in 4 segments 20 us
+// and 7 us for the merge (in 2: 43 against 36 us with the prep, in 8: 39).  The
+// merge adds a row's segments one after the other: 64 tokens at position 8000,
+// 16 x 128, 76 us in 16 segments, 67 in 32, 83 in 63.
+uint32_t prefill_seg_tiles(uint32_t n_head, uint32_t n_kv, uint32_t hd, uint32_t pos0, uint32_t batch,
+                           size_t ws_bytes) {
+  const uint32_t tq = 128u / (n_head / n_kv);
+  const size_t blocks = (size_t)n_kv * ((batch + tq - 1) / tq);
+  uint32_t seg = kSegTiles;
+  while (seg > 4u && prefill_segments(pos0, batch, seg / 2u) <= 32u &&
+         blocks * prefill_segments(pos0, batch, seg / 2u) <= 512u &&
+         prefill_part_bytes(n_head, hd, pos0, batch, seg / 2u) <= ws_bytes)
+    seg /= 2u;
+  return seg;
+}
+
+size_t attn_prefill_workspace_bytes(uint32_t n_head, uint32_t hd, uint32_t pos0, uint32_t batch) {
+  return prefill_part_bytes(n_head, hd, pos0, batch, kSegTiles);
+}
+
+// What the call uses if it may have it (at most 512 workgroups of 128 rows'
+// sums beyond attn_prefill_workspace_bytes).
+size_t attn_prefill_best_bytes(uint32_t n_head, uint32_t n_kv, uint32_t hd, uint32_t pos0, uint32_t batch) {
+  return prefill_part_bytes(n_head, hd, pos0, batch, prefill_seg_tiles(n_head, n_kv, hd, pos0, batch, ~(size_t)0));
+}
+
 hipError_t launch_attn_prefill(const KvQ8Dev& c, const float* q, const float* gate, float* out, uint32_t n_head,
-                               uint32_t pos0, uint32_t batch, void* ws, hipStream_t s) {
+                               uint32_t pos0, uint32_t batch, void* ws, size_t ws_bytes, hipStream_t s) {
   const uint32_t group = n_head / c.n_kv;
   if (group == 0 || group > kMaxGroup || batch == 0) return hipErrorInvalidValue;
   const uint32_t tq = 128u / group;
   const uint32_t blocks = (batch + tq - 1) / tq;
-  const uint32_t ns = prefill_segments(pos0, batch);
+  const uint32_t seg = prefill_seg_tiles(n_head, c.n_kv, c.hd, pos0, batch, ws_bytes);
+  const uint32_t ns = prefill_segments(pos0, batch, seg);
+  if (prefill_part_bytes(n_head, c.hd, pos0, batch, seg) > ws_bytes) return hipErrorInvalidValue;
   if (blocks > 65535u || ns > 65535u) return hipErrorInvalidValue;
   float* part = static_cast<float*>(ws);
   const dim3 grid(c.n_kv, blocks, ns);
   switch (c.hd) {
     case 32: hipLaunchKernelGGL(attn_prefill_bf16_kernel<32>, grid, dim3(256), 0, s, c, q, gate, out, part, n_head,
-                                group, tq, pos0, batch); break;
+                                group, tq, pos0, batch, seg); break;
     case 64: hipLaunchKernelGGL(attn_prefill_bf16_kernel<64>, grid, dim3(256), 0, s, c, q, gate, out, part, n_head,
-                                group, tq, pos0, batch); break;
+                                group, tq, pos0, batch, seg); break;
     case 128: hipLaunchKernelGGL(attn_prefill_bf16_kernel<128>, grid, dim3(256), 0, s, c, q, gate, out, part, n_head,
-                                 group, tq, pos0, batch); break;
+                                 group, tq, pos0, batch, seg); break;
     default: return hipErrorInvalidValue;
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || ns == 1) return e;
   const uint32_t rows = batch * n_head;
   hipLaunchKernelGGL(attn_prefill_merge_kernel, dim3((rows + 3) / 4), dim3(256), 0, s, part, c.hd, n_head, ns,
-                     kSegTiles * 32u, pos0, batch, gate, out);
+                     seg * 32u, pos0, batch, gate, out);
   return hipGetLastError();
 }
 

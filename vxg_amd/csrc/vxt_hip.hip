@@ -52,8 +52,10 @@ hipError_t launch_attn(const KvQ8Dev& c, const float* q, uint32_t n_head, uint32
 hipError_t launch_attn_step(const KvQ8Dev& c, GqaPrep pp, uint32_t rope_dim, float freq_base, float* out, void* ws,
                             hipStream_t s);
 size_t attn_prefill_workspace_bytes(uint32_t n_head, uint32_t hd, uint32_t pos0, uint32_t batch);
+size_t attn_prefill_best_bytes(uint32_t n_head, uint32_t n_kv, uint32_t hd, uint32_t pos0, uint32_t batch);
 hipError_t launch_attn_prefill(const KvQ8Dev& c, const float* q, const float* gate, float* out, uint32_t n_head,
-                               uint32_t pos0, uint32_t batch, void* ws, hipStream_t s);
+                               uint32_t pos0, uint32_t batch, void* ws, size_t ws_bytes,
+                               hipStream_t s);
 size_t greedy_state_bytes();
 hipError_t launch_greedy(const float* logits, uint32_t n, void* state, uint32_t* out, hipStream_t s);
 hipError_t launch_read_probe(const void* p, size_t bytes, uint32_t* sink, uint32_t key, hipStream_t s);
@@ -323,10 +325,14 @@ void check_matmul(Ctx* c, Tensor* t, const void* x, uint32_t x_dtype, uint32_t m
 // vxt_hip_capture_begin or the caller's own stream capture -- recorded that
 // buffer's address and may replay it later.  (Doubling bounds the kept
 // buffers by the current one.)
+bool in_capture(const Ctx* c, hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return c->capturing || (hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone);
+}
+
 void ensure_ws(Ctx* c, size_t need, hipStream_t s) {
   if (need <= c->ws_cap) return;
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  if (c->capturing || (hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone))
+  if (in_capture(c, s))
     fail(VXT_E_ARG, "workspace too small inside a capture: run this shape once before capturing");
   const size_t n = std::max(need, 2 * c->ws_cap);
   void* p = nullptr;
@@ -1118,7 +1124,12 @@ int vxt_hip_attn_step_q8_dev(void* ctx, const VxtKvQ8Cache* cache, const VxtGqaP
       const size_t per_tok = vxt::attn_prefill_workspace_bytes(n_head, kc.hd, pos, batch_m) / batch_m;
       const uint32_t group_t = (uint32_t)std::max<size_t>(
           1, std::min<size_t>(batch_m, ((size_t)256 << 20) / std::max<size_t>(per_tok, 1)));
-      ensure_ws(c, qg_bytes + per_tok * group_t, s);
+      size_t part_bytes = per_tok * group_t;
+      if (group_t == batch_m) {   // finer segments where the workspace may hold their sums
+        const size_t best = vxt::attn_prefill_best_bytes(n_head, kc.n_kv, kc.hd, pos, batch_m);
+        if (qg_bytes + best <= c->ws_cap || !in_capture(c, s)) part_bytes = std::max(part_bytes, best);
+      }
+      ensure_ws(c, qg_bytes + part_bytes, s);
       float* q_ws = static_cast<float*>(c->ws);
       a.q_out = q_ws;
       a.gate_out = params->gated_q ? q_ws + (size_t)batch_m * n_head * kc.hd : nullptr;
@@ -1128,7 +1139,7 @@ int vxt_hip_attn_step_q8_dev(void* ctx, const VxtKvQ8Cache* cache, const VxtGqaP
       for (uint32_t t = 0; t < batch_m && e == hipSuccess; t += group_t) {
         const uint32_t nb = std::min(group_t, batch_m - t);
         e = vxt::launch_attn_prefill(kc, q_ws + t * row, a.gate_out ? a.gate_out + t * row : nullptr, out + t * row,
-                                     n_head, pos + t, nb, part, s);
+                                     n_head, pos + t, nb, part, part_bytes, s);
       }
       if (e != hipSuccess) fail(VXT_E_DEVICE, std::string("prefill attention launch failed: ") + hipGetErrorString(e));
       return;
