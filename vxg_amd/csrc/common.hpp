@@ -248,19 +248,6 @@ __device__ __forceinline__ float lane_reduce(float v) {
   return v;
 }
 
-// Sum over the lanes that share lane % S (S a power of two <= 16), returned
-// in every lane: row_ror by S, 2S, .. 8 inside each 16-lane row, then across
-// rows and halves.
-template <int S>
-__device__ __forceinline__ float stride_sum(float v) {
-  if constexpr (S <= 1) v += dpp_mov<0x121>(v);   // row_ror:1
-  if constexpr (S <= 2) v += dpp_mov<0x122>(v);   // row_ror:2
-  if constexpr (S <= 4) v += dpp_mov<0x124>(v);   // row_ror:4
-  if constexpr (S <= 8) v += dpp_mov<0x128>(v);   // row_ror:8
-  v = xor16_pair(v, false);
-  return xor32_pair(v, false);
-}
-
 // Sum over the 64 lanes, returned in every lane (uniform).  DPP butterflies
 // inside each 16-lane row (quad_perm xor 1, xor 2, half-mirror, mirror), then
 // the four row sums are read out with v_readlane.  No LDS round trips.
