@@ -317,6 +317,11 @@ void check_matmul(Ctx* c, Tensor* t, const void* x, uint32_t x_dtype, uint32_t m
   if (m == 0) fail(VXT_E_SHAPE, "batch_m must be >= 1");
 }
 
+bool in_capture(const Ctx* c, hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return c->capturing || (hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone);
+}
+
 // The context workspace (GEMM weight panel and split-K partial sums, gated-FFN
 // staging, attention partial sums) is shared by every call of this context
 // (calls are ordered on one stream, or the caller orders them).  It grows only
@@ -325,11 +330,6 @@ void check_matmul(Ctx* c, Tensor* t, const void* x, uint32_t x_dtype, uint32_t m
 // vxt_hip_capture_begin or the caller's own stream capture -- recorded that
 // buffer's address and may replay it later.  (Doubling bounds the kept
 // buffers by the current one.)
-bool in_capture(const Ctx* c, hipStream_t s) {
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  return c->capturing || (hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone);
-}
-
 void ensure_ws(Ctx* c, size_t need, hipStream_t s) {
   if (need <= c->ws_cap) return;
   if (in_capture(c, s))
