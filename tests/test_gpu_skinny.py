@@ -52,3 +52,76 @@ def test_skinny_edges(eng, kind, rows, cols, M, f32):
     err = np.abs(got - want)
     assert np.all(err <= bound), float((err / bound).max())
     t.free()
+
+
+def _special_rows(m, M, cols, p, seed):
+    """N(0, 1) rows; row 0 scaled by 2^p, rows 1 .. 4 with an Inf, a -Inf (on a
+    residual's column where the matrix has some), a NaN, and Infs of both signs."""
+    X = np.random.default_rng(seed).standard_normal((M, cols)).astype(np.float32)
+    res = np.unique(m.outliers_packed & 0xFFFF) if hasattr(m, "outliers_packed") else np.zeros(0, int)
+    at = res[res.size // 2] if res.size else cols - 1
+    X[0] = np.ldexp(np.clip(X[0], -3, 3), p)
+    X[1, cols // 3] = np.inf
+    X[2, at] = -np.inf
+    X[3, cols - 2] = np.nan
+    X[min(4, M - 1), 3], X[min(4, M - 1), cols - 1] = np.inf, -np.inf
+    return X
+
+
+@pytest.mark.parametrize("kind,p", [("cb4", 124), ("g64", 124), ("q8", 120), ("q4_0", 124)])
+@pytest.mark.parametrize("rows,cols,M,f32", [
+    (70, 544, 5, False), (70, 4160, 7, False), (4200, 300, 5, False), (40, 2600, 16, False), (40, 2600, 40, False),
+    (70, 2100, 5, True), (70, 2600, 12, True), (32800, 288, 12, False)])
+def test_skinny_values_at_the_end_of_f32_and_nonfinite(eng, kind, p, rows, cols, M, f32):
+    """Outputs that f32 holds come out even where a group's or a block's sum
+    before its scale does not fit, and Inf and NaN reach the outputs that the
+    reference's loops give them to: gemv_cpu's up to 8 tokens (block dots
+    overflow there as in the reference, so Q8_0 and Q4_0 stay smaller),
+    gemm_cpu's above."""
+    print(f"skinny nonfinite {kind} rows={rows} cols={cols} M={M} f32={f32}", flush=True)
+    m = synth.make_q40(rows, cols, seed=9) if kind == "q4_0" else make(kind, rows, cols, seed=9)
+    t = eng.upload_packed(m)
+    if M <= 8 and kind in ("q8", "q4_0"):
+        p = 60
+    X = _special_rows(m, M, cols, p, cols + M)
+    xh = X if f32 else f32_to_bf16_bits(X)
+    Xq = X if f32 else bf16_bits_to_f32(xh).reshape(M, cols)
+    got = run_dev(eng, t, xh, engine.DTYPE_F32 if f32 else engine.DTYPE_BF16, M, engine.DTYPE_F32)
+    t.free()
+    W = oracle.decode_rows(m).astype(np.float64)
+    with np.errstate(all="ignore"):
+        pat = oracle.gemm(m, Xq[1:5], threads=8) if M > 8 else np.stack([oracle.gemv(m, x) for x in Xq[1:5]])
+    y = got[1:5]
+    assert np.array_equal(np.isnan(y), np.isnan(pat)) and np.array_equal(np.isinf(y), np.isinf(pat))
+    both = np.isinf(pat)
+    assert np.array_equal(np.sign(y[both]), np.sign(pat[both]))
+    fin = np.r_[0, 5:M]
+    Xf = Xq[fin].astype(np.float64)
+    want, mag = Xf @ W.T, np.abs(Xf) @ np.abs(W).T
+    assert np.abs(want).max() < 3.4e38
+    err = np.abs(got[fin] - want)
+    assert np.all(err <= (160 + cols / 128) * 2.0 ** -24 * mag)
+
+
+@pytest.mark.parametrize("kind,p", [("cb4", 124), ("q8", 120), ("q4_0", 124)])
+@pytest.mark.parametrize("cols,M", [(544, 12), (2600, 12), (544, 40)])
+def test_gated_values_at_the_end_of_f32(eng, kind, p, cols, M):
+    """The gated form on such activations: a gate far below zero gives zero
+    times a finite up, not 0 * Inf."""
+    print(f"gated end of f32 {kind} cols={cols} M={M}", flush=True)
+    F = 48
+    m = synth.make_q40(2 * F, cols, seed=9) if kind == "q4_0" else make(kind, 2 * F, cols, seed=9)
+    t = eng.upload_packed(m)
+    X = np.ldexp(np.clip(np.random.default_rng(M).standard_normal((M, cols)), -3, 3).astype(np.float32), p)
+    xh = f32_to_bf16_bits(X)
+    xd, yd = eng.to_device(xh), eng.alloc(M * F * 4)
+    eng.ffn_glu_dev(t, xd.ptr, engine.DTYPE_BF16, M, yd.ptr, engine.DTYPE_F32, F, engine.ACT_SILU, eng.stream)
+    eng.synchronize()
+    got = yd.download(np.float32, (M, F))
+    for b in (xd, yd, t):
+        b.free()
+    y = bf16_bits_to_f32(xh).reshape(M, cols).astype(np.float64) @ oracle.decode_rows(m).astype(np.float64).T
+    assert np.abs(y).max() < 3.4e38 and np.abs(y).min() > 200
+    g, u = y[:, :F], y[:, F:]
+    assert np.array_equal(got == 0, g < 0)
+    assert np.array_equal(got[g > 0], np.where(u[g > 0] > 0, np.inf, -np.inf).astype(np.float32))

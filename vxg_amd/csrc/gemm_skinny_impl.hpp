@@ -24,7 +24,8 @@
 // has three.  The product of the leading terms has accumulators of its own:
 // an infinite activation makes it infinite with the right sign while the
 // other products may be NaN (0 * Inf), so an infinite leading sum is the
-// result.
+// tile's.  An output that is not finite after all is computed anew from its
+// definition (plain_dot).
 //
 // Mapping.  A workgroup is eight waves: RG row groups of 16 weight rows by KW
 // = 8 / RG K-ways.  K is walked in phases of PH columns: the phase's
@@ -67,6 +68,7 @@
 // reads both nibbles of a byte as a pair from a 256-word table.
 #pragma once
 #include <algorithm>
+#include <type_traits>
 
 #include "act.hpp"
 #include "common.hpp"
@@ -559,6 +561,62 @@ struct Stage {
   }
 };
 
+// One output by its definition, in f64, columns [k0, k1): for a sum that came
+// out infinite or NaN.  The kernels sum a group's or a block's products before
+// its scale, so values near f32's end overflow where the result does not (cb4,
+// N(0, 1) * 2^124: 80 % of the outputs at 16 tokens), and they add cb4's
+// residuals apart, so an infinite activation at a residual's column meets two
+// weights where gemm_cpu has their sum (llm_prefill.rs:156-255).  Run by the
+// lane that stores the output, one column at a time: only for such outputs.
+// gemv: gemv_cpu's form, residuals apart and zero scales skipped
+// (codebook.rs:376-417).
+template <uint32_t KIND, int XT>
+__device__ __forceinline__ float plain_dot(const DevTensor& t, uint32_t row, const void* x, uint32_t k0, uint32_t k1,
+                                           bool gemv) {
+  auto xat = [&](uint32_t c) {
+    return XT == 3 ? static_cast<const float*>(x)[c] : bf16_to_f32(static_cast<const uint16_t*>(x)[c]);
+  };
+  const uint8_t* w = static_cast<const uint8_t*>(t.p0) + (size_t)row * (KIND == KIND_Q8 ? t.kp : t.kp / 2);
+  const uint16_t* sp = t.p1 + (size_t)row * (KIND == KIND_CB4 ? t.kp / 128 : KIND == KIND_G64 ? t.kp / 64 * 16 : t.kp / 32);
+  const float* cent = t.cent + (KIND == KIND_CB4 ? cent_table(t, row) * 16u : 0u);
+  const uint32_t os = KIND == KIND_CB4 ? t.row_ptr[row] : 0u, oe = KIND == KIND_CB4 ? t.row_ptr[row + 1] : 0u;
+  double s = 0.0;
+  for (uint32_t c = k0; c < k1 && !__builtin_isnan(s); ++c) {
+    const float xv = xat(c);
+    float v;
+    if constexpr (KIND == KIND_CB4) {
+      const float sc = f16_to_f32(sp[c / 128u]);
+      if (gemv && sc == 0.0f) continue;
+      v = sc * cent[(w[c / 2u] >> (4u * (c & 1u))) & 15u];
+      if (!gemv && !__builtin_isfinite(xv))
+        for (uint32_t i = os; i < oe; ++i)
+          if ((t.outliers[i] & 0xffffu) == c) v += f16_to_f32(t.outliers[i] >> 16);
+    } else if constexpr (KIND == KIND_G64) {
+      v = f16_to_f32(sp[(c / 64u) * 16u + ((w[c / 2u] >> (4u * (c & 1u))) & 15u)]);
+    } else if constexpr (KIND == KIND_Q40) {
+      v = (float)((int)((w[c / 32u * 16u + (c & 15u)] >> ((c & 16u) >> 2)) & 15u) - 8) * f16_to_f32(sp[c / 32u]);
+    } else {
+      v = (float)(int8_t)w[c] * f16_to_f32(sp[c / 32u]);
+    }
+    s += (double)v * (double)xv;
+  }
+  for (uint32_t i = os; i < oe; ++i) {
+    const uint32_t c = t.outliers[i] & 0xffffu;
+    const float xv = c >= k0 && c < k1 ? xat(c) : 0.0f;
+    if (c >= k0 && c < k1 && (gemv || __builtin_isfinite(xv)))
+      s += (double)f16_to_f32(t.outliers[i] >> 16) * (double)xv;
+  }
+  return (float)s;
+}
+
+// Whether an output that is not finite is computed anew.  Q8_0 and Q4_0 in
+// the GEMV's range keep the reference's block dots, which overflow as the sums
+// here do (llm_prefill.rs:45-54, q4_0.rs:109-145).
+template <uint32_t KIND>
+__device__ __forceinline__ bool redone(float v, const Args& a) {
+  return !__builtin_isfinite(v) && !((KIND == KIND_Q8 || KIND == KIND_Q40) && a.skip_zero);
+}
+
 // Decode tables shared by the workgroup (before a barrier).
 template <uint32_t KIND>
 __device__ __forceinline__ void write_tables(const DevTensor& t, uint32_t base) {
@@ -728,30 +786,43 @@ __global__ __launch_bounds__(kThreads, (MULTI ? 2 : Occ<KIND, XT, CAP, NC>)) voi
   // outputs of a tile: lanes (g, r) with g < GQ, r < WD, four tokens each
   constexpr uint32_t WD = GLU ? GH : RT, GQ = HALF ? 2 : 4, kPer = 4 * GQ * WD;
   constexpr uint32_t kOut = RG * TT * kPer;
-  for (uint32_t u = tid; u < kOut; u += kThreads) {
+  // Output u; false if it has to be redone.  The redoing pass is one of its
+  // own: it holds nothing live here.
+  auto output = [&](uint32_t u, auto redo_) {
+    constexpr bool REDO = decltype(redo_)::value;
     const uint32_t e = u % kPer, tt = u / kPer % TT, grp = u / kPer / TT;
     const uint32_t k = e / (GQ * WD), ln = e / WD % GQ * 16u + e % WD;
     const uint32_t m = tt * 16u + 4u * (ln >> 4) + k;
-    if (m >= M) continue;
+    const uint32_t o = blockIdx.x * ((GLU ? GH : RT) * RG) + (GLU ? GH : RT) * grp + (ln & 15u);
+    const uint32_t lim = GLU ? a.y_stride : t.rows;
+    if (m >= M || o >= lim) return true;
+    const void* xm = static_cast<const char*>(a.x) + (size_t)m * t.cols * (XT == 3 ? 4u : 2u);
     float v = total(grp, tt, k, ln);
-    uint32_t o, lim;
+    bool ok = !redone<KIND>(v, a);
+    if (REDO && !ok) v = plain_dot<KIND, XT>(t, o, xm, k0, cols, a.skip_zero != 0);
     if constexpr (GLU) {
-      const float up = total(grp, tt, k, ln + GH);
-      o = blockIdx.x * (GH * RG) + GH * grp + (ln & 15u);
-      lim = a.y_stride;
-      v = o < a.n_ff ? gated_act(v, up, a.gelu != 0) : 0.0f;   // zero padding up to the row stride
-    } else {
-      o = blockIdx.x * (RT * RG) + RT * grp + (ln & 15u);
-      lim = t.rows;
+      float up = total(grp, tt, k, ln + GH);
+      const bool up_ok = !redone<KIND>(up, a);
+      if (o >= a.n_ff) {
+        v = 0.0f;   // zero padding up to the row stride
+        ok = true;
+      } else {
+        if (REDO && !up_ok) up = plain_dot<KIND, XT>(t, a.n_ff + o, xm, k0, cols, a.skip_zero != 0);
+        ok = ok && up_ok;
+        v = gated_act(v, up, a.gelu != 0);
+      }
     }
-    if (o < lim) {
-      const size_t at = (size_t)m * lim + o;
-      if (a.y_bf16)
-        static_cast<uint16_t*>(a.y)[at] = f32_to_bf16(v);
-      else
-        static_cast<float*>(a.y)[at] = v;
-    }
-  }
+    const size_t at = (size_t)m * lim + o;
+    if (a.y_bf16)
+      static_cast<uint16_t*>(a.y)[at] = f32_to_bf16(v);
+    else
+      static_cast<float*>(a.y)[at] = v;
+    return ok;
+  };
+  bool ok = true;
+  for (uint32_t u = tid; u < kOut; u += kThreads) ok = output(u, std::false_type{}) && ok;
+  if (__builtin_expect(!ok, 0))
+    for (uint32_t u = tid; u < kOut; u += kThreads) output(u, std::true_type{});
 }
 
 // Many rows (an LM head): each wave streams whole 16-row tiles, wv, wv +
@@ -842,16 +913,26 @@ __global__ __launch_bounds__(kThreads, 4) void skinny_stream_kernel(DevTensor t,
     tile.accl[0] = tl;
     if constexpr (KIND == KIND_CB4)
       tile.template residuals<1, KP>(t.outliers, pre, os, oe, 0, M, xoff, XS, 0, PH);
+    const uint32_t o = ti * 16u + r;
+    auto store = [&](uint32_t m, float v) {
+      const size_t at = (size_t)m * rows + o;
+      if (a.y_bf16)
+        static_cast<uint16_t*>(a.y)[at] = f32_to_bf16(v);
+      else
+        static_cast<float*>(a.y)[at] = v;
+    };
+    uint32_t redo = 0;
 #pragma unroll
     for (uint32_t k = 0; k < 4; ++k) {
-      const uint32_t m = 4u * g + k, o = ti * 16u + r;
-      if (m < M && o < rows) {
-        const size_t at = (size_t)m * rows + o;
-        if (a.y_bf16)
-          static_cast<uint16_t*>(a.y)[at] = f32_to_bf16(tile.sum(0, k));
-        else
-          static_cast<float*>(a.y)[at] = tile.sum(0, k);
+      const float v = tile.sum(0, k);
+      if (4u * g + k < M && o < rows) {
+        store(4u * g + k, v);
+        redo |= redone<KIND>(v, a) ? 1u << k : 0u;
       }
+    }
+    for (; __builtin_expect(redo != 0, 0); redo &= redo - 1u) {
+      const uint32_t m = 4u * g + (uint32_t)__builtin_ctz(redo);
+      store(m, plain_dot<KIND, 1>(t, o, static_cast<const uint16_t*>(a.x) + (size_t)m * cols, 0, cols, a.skip_zero != 0));
     }
   }
 }
