@@ -125,3 +125,40 @@ def test_gated_values_at_the_end_of_f32(eng, kind, p, cols, M):
     g, u = y[:, :F], y[:, F:]
     assert np.array_equal(got == 0, g < 0)
     assert np.array_equal(got[g > 0], np.where(u[g > 0] > 0, np.inf, -np.inf).astype(np.float32))
+
+
+@pytest.mark.parametrize("kind", ["cb4", "g64", "q8", "q4_0"])
+@pytest.mark.parametrize("rows,cols,M", [(70, 544, 3), (40, 2600, 7), (40, 2100, 12)])
+def test_skinny_f32_activations_near_the_small_end(eng, kind, rows, cols, M):
+    """f32 activations down to the subnormals keep all their bits.  Beyond the
+    file's bound an output has an absolute error of at most half of f32's
+    smallest step (2^-150) per product and per sum, before a scale below 1."""
+    print(f"skinny small f32 {kind} rows={rows} cols={cols} M={M}", flush=True)
+    m = synth.make_q40(rows, cols, seed=4) if kind == "q4_0" else make(kind, rows, cols, seed=4)
+    t = eng.upload_packed(m)
+    X = np.random.default_rng(M).standard_normal((M, cols))
+    X = (X * np.exp2(np.linspace(-100, -136, M))[:, None]).astype(np.float32)
+    got = run_dev(eng, t, X, engine.DTYPE_F32, M, engine.DTYPE_F32)
+    t.free()
+    W = oracle.decode_rows(m).astype(np.float64)
+    want, mag = X.astype(np.float64) @ W.T, np.abs(X).astype(np.float64) @ np.abs(W).T
+    err = np.abs(got - want)
+    assert np.all(err <= (160 + cols / 128) * 2.0 ** -24 * mag + 2 * cols * 2.0 ** -150)
+
+
+def test_skinny_small_centroids(eng):
+    """Centroids near f32's small end keep all their bits: the table times
+    2^-118, against the same products times 2^-118."""
+    rows, cols, M = 70, 544, 6
+    m = synth.make_cb4(rows, cols, seed=4, outlier_frac=0.0)
+    W = oracle.decode_rows(m).astype(np.float64)
+    m.centroids[:] = np.ldexp(m.centroids, -118)
+    t = eng.upload_packed(m)
+    X = np.full((M, cols), np.ldexp(1.0, 100), np.float32)
+    X[1:] *= np.random.default_rng(M).standard_normal((M - 1, cols)).astype(np.float32)
+    X = bf16_bits_to_f32(f32_to_bf16_bits(X)).reshape(M, cols)
+    got = run_dev(eng, t, f32_to_bf16_bits(X), engine.DTYPE_BF16, M, engine.DTYPE_F32)
+    t.free()
+    want = np.ldexp(X.astype(np.float64) @ W.T, -118)
+    rel = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
+    assert rel.max() <= 4 * 2.0 ** -24, rel      # the sums' own error is 0.7 .. 0.9e-7; lost centroid bits gave 2^-15

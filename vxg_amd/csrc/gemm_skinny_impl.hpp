@@ -11,7 +11,9 @@
 // the products go to v_mfma_f32_16x16x32_bf16: 16 tokens (A, rows past the
 // batch repeat the last one and are never stored) by 16 weight rows (B).
 //
-// Exact operands.  bf16 has f32's range, so no operand needs a scale:
+// Exact operands.  bf16 has f32's range, so no operand needs a scale; a second
+// term of an f32 value is kept times 2^8 and a third times 2^16, as bf16 ends at
+// 2^-133 and f32 at 2^-149 (unscaled, activations of 2^-126 came out 4.5e-3 off):
 //   * g64: an f16 table entry is two bf16 terms (8 + 3 significant bits);
 //   * cb4: an f32 centroid is three (8 + 8 + 8 bits); a 128-column group's
 //     products are summed in fresh accumulators and scaled once, as the
@@ -101,16 +103,16 @@ constexpr int kThreads = 64 * kWaves;
 constexpr uint32_t kStreamRows = 32768;
 constexpr uint32_t kHalfRows = 4096;
 
-// f32 as three bf16 terms (bits in the high halves): v = h + m + l exactly.
-// Inf and NaN are h alone.
+// f32 as three bf16 terms, each the high half of a word (what the low halves
+// hold is not read): v = h + m 2^-8 + l 2^-16 exactly, subnormals too.  Inf and
+// NaN are h alone; canonicalising sets a NaN's quiet bit, so the cut keeps it one.
+constexpr float kTerm1 = 1.0f / 256.0f, kTerm2 = 1.0f / 65536.0f;
 __device__ __forceinline__ void split3(float v, uint32_t& h, uint32_t& m, uint32_t& l) {
-  const uint32_t b = __float_as_uint(v);
-  const bool fin = (b & 0x7f800000u) != 0x7f800000u;
-  h = b & 0xffff0000u;
-  if ((b & 0x7fffffffu) > 0x7f800000u) h |= 0x00400000u;   // a NaN's payload may lie in the cut bits
-  const float r = fin ? v - __uint_as_float(h) : 0.0f;
-  m = __float_as_uint(r) & 0xffff0000u;
-  l = __float_as_uint(r - __uint_as_float(m)) & 0xffff0000u;
+  auto cut = [](float f) { return __uint_as_float(__float_as_uint(f) & 0xffff0000u); };
+  const float r = __builtin_isfinite(v) ? (v - cut(v)) * 256.0f : 0.0f;
+  h = __float_as_uint(__builtin_canonicalizef(v));
+  m = __float_as_uint(r);
+  l = __float_as_uint((r - cut(r)) * 256.0f);
 }
 
 __device__ __forceinline__ uint32_t lo_pair(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x05040100u); }
@@ -191,10 +193,11 @@ struct Tile {
   }
 
   // One MFMA step: the B terms against the activations at column position c.
-  // The lesser products alternate between two accumulators: a wave's chain of
-  // dependent MFMAs is half as long.
+  // The lesser products go to an accumulator for each power of 2^-8 that the
+  // terms' products carry (g64's two terms carry none), 2^-24 in lo[0]: shorter
+  // chains of dependent MFMAs too.
   template <int WT>
-  __device__ __forceinline__ void step(const bf16x8_t (&b)[WT], uint32_t c, f32x4_t (&hi)[TT], f32x4_t (&lo)[2][TT]) {
+  __device__ __forceinline__ void step(const bf16x8_t (&b)[WT], uint32_t c, f32x4_t (&hi)[TT], f32x4_t (&lo)[3][TT]) {
 #pragma unroll
     for (int i = 0; i < TT; ++i) {
 #pragma unroll
@@ -206,12 +209,19 @@ struct Tile {
           if (wt + xt == 0) {
             hi[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, b[wt], hi[i], 0, 0, 0);
           } else {
-            f32x4_t& l = lo[(wt + xt) & 1][i];
+            f32x4_t& l = lo[((KIND == KIND_CB4 ? wt : 0) + xt) % 3][i];
             l = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, b[wt], l, 0, 0, 0);
           }
         }
       }
     }
+  }
+
+  // The lesser products' sum of a chunk; sums that were never formed stay out.
+  __device__ __forceinline__ float lesser(const f32x4_t (&lo)[3][TT], int i, int k) const {
+    float v = KIND == KIND_G64 ? lo[0][i][k] : KIND == KIND_CB4 && XT > 1 ? lo[0][i][k] * (kTerm1 * kTerm2) : 0.0f;
+    if constexpr (KIND == KIND_CB4 || XT > 1) v = __builtin_fmaf(lo[1][i][k], kTerm1, __builtin_fmaf(lo[2][i][k], kTerm2, v));
+    return v;
   }
 
   // Weights of columns past the row's end, zeroed: an Inf or NaN there must
@@ -230,9 +240,9 @@ struct Tile {
     constexpr uint32_t CH = kChunk<KIND>;
     const f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
     if constexpr (KIND == KIND_CB4) {
-      f32x4_t fh[TT], fl[2][TT];
+      f32x4_t fh[TT], fl[3][TT];
 #pragma unroll
-      for (int i = 0; i < TT; ++i) fh[i] = fl[0][i] = fl[1][i] = z;
+      for (int i = 0; i < TT; ++i) fh[i] = fl[0][i] = fl[1][i] = fl[2][i] = z;
       const uint32_t wd[4] = {w.q.x, w.q.y, w.q.z, w.q.w};
 #pragma unroll
       for (uint32_t j = 0; j < 4; ++j) {
@@ -262,7 +272,7 @@ struct Tile {
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
           acc[i][k] = skip ? acc[i][k] : __builtin_fmaf(s, fh[i][k], acc[i][k]);
-          accl[i][k] = skip ? accl[i][k] : __builtin_fmaf(s, fl[0][i][k] + fl[1][i][k], accl[i][k]);
+          accl[i][k] = skip ? accl[i][k] : __builtin_fmaf(s, lesser(fl, i, k), accl[i][k]);
         }
     } else if constexpr (KIND == KIND_G64) {
       // the lane's table: two terms of each f16 entry in one word
@@ -280,9 +290,9 @@ struct Tile {
       // a table word's address: byte 0 the lane's column, byte 1 the block and the nibble
       const uint32_t lbyte = lane * 4u, rep = ((tab >> 8) & 0xffu) * 0x01010101u;
       const uint32_t wd[8] = {w.q0.x, w.q0.y, w.q0.z, w.q0.w, w.q1.x, w.q1.y, w.q1.z, w.q1.w};
-      f32x4_t fh[2][TT], fl[2][TT];   // two chains of leading products: half the roundings in a row
+      f32x4_t fh[2][TT], fl[3][TT];   // two chains of leading products: half the roundings in a row
 #pragma unroll
-      for (int i = 0; i < TT; ++i) fh[0][i] = fh[1][i] = fl[0][i] = fl[1][i] = z;
+      for (int i = 0; i < TT; ++i) fh[0][i] = fh[1][i] = fl[0][i] = fl[1][i] = fl[2][i] = z;
 #pragma unroll
       for (uint32_t j = 0; j < 8; ++j) {
         const uint32_t we = (wd[j] & 0x0F0F0F0Fu) | rep, wo = ((wd[j] >> 4) & 0x0F0F0F0Fu) | rep;
@@ -309,7 +319,7 @@ struct Tile {
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
           acc[i][k] += fh[0][i][k] + fh[1][i][k];
-          accl[i][k] += XT == 1 ? fl[1][i][k] : fl[0][i][k] + fl[1][i][k];
+          accl[i][k] += lesser(fl, i, k);
         }
     } else {
       // Blocks past the row hold a repeated block: scale 0 (its products are
@@ -353,9 +363,9 @@ struct Tile {
         }
         const u32x4 v = {d[0], d[1], d[2], d[3]};
         const bf16x8_t b[1] = {__builtin_bit_cast(bf16x8_t, v)};
-        f32x4_t fh[TT], fl[2][TT];
+        f32x4_t fh[TT], fl[3][TT];
 #pragma unroll
-        for (int i = 0; i < TT; ++i) fh[i] = fl[0][i] = fl[1][i] = z;
+        for (int i = 0; i < TT; ++i) fh[i] = fl[0][i] = fl[1][i] = fl[2][i] = z;
         step(b, at + 32u * j + 8u * g, fh, fl);
         const float s = f16_to_f32(s4[j]);
 #pragma unroll
@@ -363,7 +373,7 @@ struct Tile {
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
             ch[i][k] = __builtin_fmaf(s, fh[i][k], ch[i][k]);
-            if constexpr (XT > 1) cl[i][k] = __builtin_fmaf(s, fl[0][i][k] + fl[1][i][k], cl[i][k]);
+            if constexpr (XT > 1) cl[i][k] = __builtin_fmaf(s, lesser(fl, i, k), cl[i][k]);
           }
       }
 #pragma unroll
@@ -413,7 +423,8 @@ struct Tile {
             xv[j] = 0.0f;
 #pragma unroll
             for (int xt = XT - 1; xt >= 0; --xt)   // the terms' sum is exact, smallest first
-              xv[j] += bf16_to_f32(*(lds_u16*)(size_t)(at[j] + xt * plane + m * xs));
+              xv[j] = __builtin_fmaf(bf16_to_f32(*(lds_u16*)(size_t)(at[j] + xt * plane + m * xs)),
+                                     xt == 2 ? kTerm2 : xt == 1 ? kTerm1 : 1.0f, xv[j]);
           }
 #pragma unroll
           for (int j = 0; j < 4; ++j) accr[tt][i] = on[j] ? __builtin_fmaf(v[j], xv[j], accr[tt][i]) : accr[tt][i];
