@@ -558,7 +558,9 @@ VXT_API int vxt_hip_last_kernel_ms(void* ctx, double* ms);
 /* Prefill GEMM path (batch_m > 8) of this context's later calls.  Every path
  * runs this library's own kernels except LIBRARY.  AUTO (the default), by
  * measured speed: every kind takes the few-token MFMA kernels up to batch_m
- * 16, and to 32 or 64 by kind and size; above, g64 weights with bf16
+ * 16 (unless their partial sums need more than the workspace of the other
+ * paths: g64 and Q8_0 of many rows and cols > 2048), and to 32 or 64 by kind
+ * and size; above, g64 weights with bf16
  * activations decode inside the MFMA loop -- the fused kernel up to batch_m 64,
  * the 128 x 128 tile kernel above, to 767 (1023 when cols > rows); cb4 weights with bf16
  * activations take the cb4 tile kernel described under FUSED from batch_m 128

@@ -62,6 +62,29 @@ def test_noalloc_matches_matmul_dev_on_two_calls(eng, kind, rows, cols, xdt, m1,
     t.free()
 
 
+@pytest.mark.parametrize("kind,rows,cols,M", [("q8", 32768, 2112, 16), ("g64", 12288, 8192, 9), ("q8", 4096, 4160, 12)])
+def test_a_call_does_not_depend_on_the_workspace(kind, rows, cols, M):
+    """Shapes whose few-token K ranges need more workspace than the other
+    paths reserve (and one that needs less): the first call of a context, the
+    same call after a larger one has grown the workspace, and the
+    allocation-free entry point give the same bits."""
+    print(f"workspace independence kind={kind} {rows}x{cols} M={M}", flush=True)
+    e = engine.HipEngine(0)
+    try:
+        t = e.upload_packed({"g64": synth.make_g64, "q8": synth.make_q8}[kind](rows, cols, seed=M))
+        xh = synth.make_x_bf16(M, cols, seed=M)
+        first, noalloc = both(e, t, xh, engine.DTYPE_BF16, M)
+        big = e.upload_packed(synth.make_q8(2048, 2048, seed=1))
+        grow = synth.make_x_f32(2048, 2048, seed=1)
+        xd, yd = e.to_device(grow), e.alloc(2048 * 2048 * 4)
+        e.matmul_dev(big, xd.ptr, engine.DTYPE_F32, 2048, yd.ptr, engine.DTYPE_F32, e.stream)
+        again, noalloc2 = both(e, t, xh, engine.DTYPE_BF16, M)
+        for y in (noalloc, again, noalloc2):
+            assert_bits_equal(y, first)
+    finally:
+        e.close()
+
+
 def test_noalloc_in_a_graph_without_a_sizing_call():
     """A fresh context: the first call of this shape is captured (matmul_dev
     would refuse to grow its workspace there); replays equal the eager

@@ -1255,7 +1255,7 @@ static size_t path_workspace_bytes(Path path, const DevTensor& t, uint32_t m, bo
 }
 
 // The few-token kernels (gemm_skinny.hip) take a call in AUTO up to 16 tokens
-// always, and up to 32 and 64 while each weight's decode, repeated for every
+// (within the workspace rule of takes_skinny), and up to 32 and 64 while each weight's decode, repeated for every
 // 32 tokens, is cheaper than a panel, as measured by kind (whole call, us,
 // this against the general path; K -> N):
 //   M = 17..32: cb4, Q4_0 always (32 tokens 2048 -> 6144 15.7 / 11.6 against
@@ -1284,14 +1284,9 @@ bool skinny_takes(const DevTensor& t, uint32_t m, bool x_bf16) {
   }
 }
 
-static bool takes_skinny(const DevTensor& t, uint32_t m, bool x_bf16, int mode, size_t general_bytes) {
-  return (mode == kGemmAuto || mode == kGemmAutoOwn) && skinny_takes(t, m, x_bf16) &&
-         skinny_workspace_bytes(t, m, x_bf16) <= general_bytes;
-}
-
 // The general path's workspace, also for a call that the few-token kernels
-// take (they need less): which calls fit a capture, or the allocation-free
-// entry point's scratch, does not depend on that choice.
+// take: which calls fit a capture, or the allocation-free entry point's
+// scratch, does not depend on that choice.
 size_t gemm_workspace_bytes(const DevTensor& t, uint32_t m, bool x_bf16, int mode) {
   const Path path = general_path(t, m, x_bf16, mode);
   size_t n = path_workspace_bytes(path, t, m, x_bf16, mode);
@@ -1301,11 +1296,24 @@ size_t gemm_workspace_bytes(const DevTensor& t, uint32_t m, bool x_bf16, int mod
   return n;
 }
 
+// The few-token kernels' K ranges can need more than that (g64 and Q8_0, whose
+// fused kernel may have no partial sums: 16 tokens at K = 2112 .. 4096 from
+// 32768 rows, 8192 from 12288): such a call keeps the general path.  The choice
+// looks at what the call reserves, not at what the workspace has grown to, so a
+// call's kernel, and its bits, do not depend on the calls before it.
+static bool takes_skinny(const DevTensor& t, uint32_t m, bool x_bf16, int mode) {
+  return (mode == kGemmAuto || mode == kGemmAutoOwn) && skinny_takes(t, m, x_bf16) &&
+         skinny_workspace_bytes(t, m, x_bf16) <= gemm_workspace_bytes(t, m, x_bf16, mode);
+}
+
 hipError_t launch_gemm(const DevTensor& t, const void* x, bool x_bf16, uint32_t m, void* y, bool y_bf16, void* ws,
                        size_t ws_bytes, hipStream_t s, int mode) {
   if (m == 0 || (size_t)m * t.rows > (size_t)1 << 40) return hipErrorInvalidValue;
+  if (takes_skinny(t, m, x_bf16, mode)) {
+    if (ws_bytes < skinny_workspace_bytes(t, m, x_bf16)) return hipErrorInvalidValue;
+    return launch_skinny(t, x, x_bf16, m, y, y_bf16, ws, s);
+  }
   const Path path = general_path(t, m, x_bf16, mode);
-  if (takes_skinny(t, m, x_bf16, mode, ws_bytes)) return launch_skinny(t, x, x_bf16, m, y, y_bf16, ws, s);
   if (path == Path::Tile)
     return launch_gemm_tile(t, static_cast<const uint16_t*>(x), m, y, y_bf16, ws, ws_bytes, s);
   if (path == Path::TileCb4)
