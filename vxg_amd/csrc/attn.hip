@@ -1157,8 +1157,9 @@ hipError_t launch_attn(const KvQ8Dev& c, const float* q, uint32_t n_head, uint32
 // Causal attention of batch prepared queries (q, gate: [batch][n_head][hd])
 // on MFMA: tokens at positions pos0 .. pos0 + batch - 1, every cache row up to
 // the last written.  hd <= 128.  Positions are cut into segments of
-// seg_tiles * 32 when there are more than one; ws then holds
-// prefill_part_bytes(...) of partial sums.
+// seg_tiles * 32 when there are more than one; their sums go to ws
+// (attn_prefill_workspace_bytes(...)) for segments of kSegTiles, to split
+// (kAttnSplitBytes) for shorter ones.
 uint32_t prefill_segments(uint32_t pos0, uint32_t batch, uint32_t seg_tiles) {
   return (pos0 + batch - 1u) / (seg_tiles * 32u) + 1u;
 }
@@ -1169,21 +1170,23 @@ size_t prefill_part_bytes(uint32_t n_head, uint32_t hd, uint32_t pos0, uint32_t 
 }
 
 // The segment length: kSegTiles, halved down to 4 tiles while the grid stays
-// within the 512 workgroups that run at once, a token has at most 32 segments
-// and the partial sums fit ws_bytes.  A workgroup walks its tiles one after the
+// within the 512 workgroups that run at once and a token has at most 32
+// segments.  The call alone decides (a capture gives the eager call's result).
+// A workgroup walks its tiles one after the
 // other, about 3 us each, and a short prompt has few of them: 500 tokens, 16
 // heads x 128, are 64 workgroups of up to 16 tiles, 52 us; in 4 segments 20 us
 // and 7 us for the merge (in 2: 43 against 36 us with the prep, in 8: 39).  The
 // merge adds a row's segments one after the other: 64 tokens at position 8000,
 // 16 x 128, 76 us in 16 segments, 67 in 32, 83 in 63.
-uint32_t prefill_seg_tiles(uint32_t n_head, uint32_t n_kv, uint32_t hd, uint32_t pos0, uint32_t batch,
-                           size_t ws_bytes) {
+constexpr uint32_t kMaxSplitBlocks = 512;
+// A workgroup of a shorter segment holds at most 128 rows' sums.
+static_assert(kAttnSplitBytes == (size_t)kMaxSplitBlocks * 128 * (128 + 2) * sizeof(float), "split buffer");
+uint32_t prefill_seg_tiles(uint32_t n_head, uint32_t n_kv, uint32_t pos0, uint32_t batch) {
   const uint32_t tq = 128u / (n_head / n_kv);
   const size_t blocks = (size_t)n_kv * ((batch + tq - 1) / tq);
   uint32_t seg = kSegTiles;
   while (seg > 4u && prefill_segments(pos0, batch, seg / 2u) <= 32u &&
-         blocks * prefill_segments(pos0, batch, seg / 2u) <= 512u &&
-         prefill_part_bytes(n_head, hd, pos0, batch, seg / 2u) <= ws_bytes)
+         blocks * prefill_segments(pos0, batch, seg / 2u) <= kMaxSplitBlocks)
     seg /= 2u;
   return seg;
 }
@@ -1192,20 +1195,18 @@ size_t attn_prefill_workspace_bytes(uint32_t n_head, uint32_t hd, uint32_t pos0,
   return prefill_part_bytes(n_head, hd, pos0, batch, kSegTiles);
 }
 
-// What the call uses if it may have it (at most 512 workgroups of 128 rows'
-// sums beyond attn_prefill_workspace_bytes).
-size_t attn_prefill_best_bytes(uint32_t n_head, uint32_t n_kv, uint32_t hd, uint32_t pos0, uint32_t batch) {
-  return prefill_part_bytes(n_head, hd, pos0, batch, prefill_seg_tiles(n_head, n_kv, hd, pos0, batch, ~(size_t)0));
-}
-
 hipError_t launch_attn_prefill(const KvQ8Dev& c, const float* q, const float* gate, float* out, uint32_t n_head,
-                               uint32_t pos0, uint32_t batch, void* ws, size_t ws_bytes, hipStream_t s) {
+                               uint32_t pos0, uint32_t batch, void* ws, size_t ws_bytes, void* split, hipStream_t s) {
   const uint32_t group = n_head / c.n_kv;
   if (group == 0 || group > kMaxGroup || batch == 0) return hipErrorInvalidValue;
   const uint32_t tq = 128u / group;
   const uint32_t blocks = (batch + tq - 1) / tq;
-  const uint32_t seg = prefill_seg_tiles(n_head, c.n_kv, c.hd, pos0, batch, ws_bytes);
+  const uint32_t seg = prefill_seg_tiles(n_head, c.n_kv, pos0, batch);
   const uint32_t ns = prefill_segments(pos0, batch, seg);
+  if (seg < kSegTiles) {
+    ws = split;
+    ws_bytes = kAttnSplitBytes;
+  }
   if (prefill_part_bytes(n_head, c.hd, pos0, batch, seg) > ws_bytes) return hipErrorInvalidValue;
   if (blocks > 65535u || ns > 65535u) return hipErrorInvalidValue;
   float* part = static_cast<float*>(ws);

@@ -53,6 +53,10 @@ enum GemmMode : int { kGemmAuto = 0, kGemmPanel = 1, kGemmFused = 2, kGemmLibrar
 // Bytes of the scratch array of the allocation-free matmul entry point.
 constexpr size_t kNoAllocScratch = (size_t)32 << 20;
 
+// Bytes of a context's buffer for the sums of prefill attention's shorter
+// position segments: 512 workgroups x 128 rows x (128 + 2) floats.
+constexpr size_t kAttnSplitBytes = (size_t)512 * 128 * (128 + 2) * 4;
+
 // Centroid table serving `row` (rows of up to 3 concatenated sub-matrices).
 __device__ __forceinline__ uint32_t cent_table(const DevTensor& t, uint32_t row) {
   return (uint32_t)(row >= t.split0) + (uint32_t)(row >= t.split1);

@@ -52,10 +52,8 @@ hipError_t launch_attn(const KvQ8Dev& c, const float* q, uint32_t n_head, uint32
 hipError_t launch_attn_step(const KvQ8Dev& c, GqaPrep pp, uint32_t rope_dim, float freq_base, float* out, void* ws,
                             hipStream_t s);
 size_t attn_prefill_workspace_bytes(uint32_t n_head, uint32_t hd, uint32_t pos0, uint32_t batch);
-size_t attn_prefill_best_bytes(uint32_t n_head, uint32_t n_kv, uint32_t hd, uint32_t pos0, uint32_t batch);
 hipError_t launch_attn_prefill(const KvQ8Dev& c, const float* q, const float* gate, float* out, uint32_t n_head,
-                               uint32_t pos0, uint32_t batch, void* ws, size_t ws_bytes,
-                               hipStream_t s);
+                               uint32_t pos0, uint32_t batch, void* ws, size_t ws_bytes, void* split, hipStream_t s);
 size_t greedy_state_bytes();
 hipError_t launch_greedy(const float* logits, uint32_t n, void* state, uint32_t* out, hipStream_t s);
 hipError_t launch_read_probe(const void* p, size_t bytes, uint32_t* sink, uint32_t key, hipStream_t s);
@@ -134,6 +132,7 @@ struct Ctx {
   void* ws = nullptr;           // workspace: GEMM panel, partial sums, staging
   size_t ws_cap = 0;
   std::vector<void*> retired;   // replaced workspaces, kept until destroy
+  void* attn_split = nullptr;   // sums of prefill attention's shorter segments (kAttnSplitBytes)
   void* greedy = nullptr;  // greedy-selection state words (zero between calls)
   void* scratch = nullptr; // device address of `scratch` on this context's device
   int gemm_mode = vxt::kGemmAuto;
@@ -391,11 +390,13 @@ void* vxt_hip_create(int32_t device, char* dev_name, size_t dev_name_cap, char* 
       VXT_HIP_CHECK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
       VXT_HIP_CHECK(hipEventCreate(&c->ev0));
       VXT_HIP_CHECK(hipEventCreate(&c->ev1));
+      VXT_HIP_CHECK(hipMalloc(&c->attn_split, vxt::kAttnSplitBytes));
       VXT_HIP_CHECK(hipMalloc(&c->greedy, vxt::greedy_state_bytes()));
       VXT_HIP_CHECK(hipMemset(c->greedy, 0, vxt::greedy_state_bytes()));
       VXT_HIP_CHECK(hipGetSymbolAddress(&c->scratch, HIP_SYMBOL(scratch)));   // with `dev` current
     } catch (...) {
       if (c->greedy) (void)hipFree(c->greedy);
+      if (c->attn_split) (void)hipFree(c->attn_split);
       if (c->ev1) (void)hipEventDestroy(c->ev1);
       if (c->ev0) (void)hipEventDestroy(c->ev0);
       if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -445,6 +446,7 @@ void vxt_hip_destroy(void* ctx) {
   if (c->ws) (void)hipFree(c->ws);
   for (void* b : c->retired) (void)hipFree(b);
   if (c->greedy) (void)hipFree(c->greedy);
+  if (c->attn_split) (void)hipFree(c->attn_split);
   (void)hipEventDestroy(c->ev0);
   (void)hipEventDestroy(c->ev1);
   (void)hipStreamDestroy(c->stream);
@@ -1124,11 +1126,7 @@ int vxt_hip_attn_step_q8_dev(void* ctx, const VxtKvQ8Cache* cache, const VxtGqaP
       const size_t per_tok = vxt::attn_prefill_workspace_bytes(n_head, kc.hd, pos, batch_m) / batch_m;
       const uint32_t group_t = (uint32_t)std::max<size_t>(
           1, std::min<size_t>(batch_m, ((size_t)256 << 20) / std::max<size_t>(per_tok, 1)));
-      size_t part_bytes = per_tok * group_t;
-      if (group_t == batch_m) {   // finer segments where the workspace may hold their sums
-        const size_t best = vxt::attn_prefill_best_bytes(n_head, kc.n_kv, kc.hd, pos, batch_m);
-        if (qg_bytes + best <= c->ws_cap || !in_capture(c, s)) part_bytes = std::max(part_bytes, best);
-      }
+      const size_t part_bytes = per_tok * group_t;
       ensure_ws(c, qg_bytes + part_bytes, s);
       float* q_ws = static_cast<float*>(c->ws);
       a.q_out = q_ws;
@@ -1139,7 +1137,7 @@ int vxt_hip_attn_step_q8_dev(void* ctx, const VxtKvQ8Cache* cache, const VxtGqaP
       for (uint32_t t = 0; t < batch_m && e == hipSuccess; t += group_t) {
         const uint32_t nb = std::min(group_t, batch_m - t);
         e = vxt::launch_attn_prefill(kc, q_ws + t * row, a.gate_out ? a.gate_out + t * row : nullptr, out + t * row,
-                                     n_head, pos + t, nb, part, part_bytes, s);
+                                     n_head, pos + t, nb, part, part_bytes, c->attn_split, s);
       }
       if (e != hipSuccess) fail(VXT_E_DEVICE, std::string("prefill attention launch failed: ") + hipGetErrorString(e));
       return;
