@@ -271,3 +271,33 @@ def test_tile_kernel_one_round_grids(eng, M, N, K):
     b = check(eng, synth.make_g64(N, K, seed=M + N), M, engine.GEMM_FUSED, seed=K)
     assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
     check(eng, make("cb4", N, K, seed=M + N), M, engine.GEMM_FUSED, seed=K)
+
+
+# Two or one K slices in place of three or two: each way's first half is summed
+# apart.  Ways of 2 to 16 tiles (a half of none, an odd count, a way that ends
+# a tile early), ragged M, N and K.  bar: the relative error of one slice more,
+# in the order below 1.29, 1.82, 1.52 and 2.21e-7, and 2 % (without the halves
+# 1.52, 2.17, 2.08 and 2.40e-7).
+@pytest.mark.parametrize("kind,M,N,K,bar", [
+    ("g64", 200, 6144, 2048, 1.32e-7), ("cb4", 200, 6144, 2048, 1.86e-7), ("g64", 300, 6144, 2048, 1.56e-7),
+    ("cb4", 300, 2048, 6144, 2.25e-7), ("g64", 300, 6100, 512, None), ("g64", 290, 5900, 700, None),
+    ("g64", 200, 6000, 1100, None), ("cb4", 300, 6100, 256, None), ("cb4", 300, 5900, 700, None)])
+def test_tile_kernels_sums_in_halves(eng, kind, M, N, K, bar):
+    print(f"tile halves {kind} M={M} N={N} K={K}", flush=True)
+    m = synth.make_g64(N, K, seed=5) if kind == "g64" else make(kind, N, K, seed=5)
+    t = eng.upload_packed(m)
+    xb = synth.make_x_bf16(M, K, seed=M)
+    X = bf16_bits_to_f32(xb).reshape(M, K).astype(np.float64)
+    eng.set_gemm_path(engine.GEMM_FUSED)
+    try:
+        got = run_dev(eng, t, xb, engine.DTYPE_BF16, M, engine.DTYPE_F32)
+    finally:
+        eng.set_gemm_path(engine.GEMM_AUTO)
+    t.free()
+    W = oracle.decode_rows(m).astype(np.float64)
+    want = X @ W.T
+    # K / 16 sums of 16 exact products in a row at most, each within 2^-24 of the terms' magnitudes (cb4's table
+    # entries are exact to 2^-22)
+    assert np.all(np.abs(got - want) <= (K / 16 + 20) * 2.0 ** -24 * (np.abs(X) @ np.abs(W).T))
+    if bar:
+        assert np.linalg.norm(got - want) / np.linalg.norm(want) <= bar

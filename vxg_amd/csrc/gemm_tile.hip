@@ -282,7 +282,9 @@ template <int KW>
 constexpr size_t lds_bytes() { return out_offset<KW>() + (size_t)BM * LDO * 2; }
 
 // gridDim.x = tiles_m * tiles_n, gridDim.y = K slices of kt_per_split tiles.
-template <int KW>
+// FOLD: a way's first half is summed apart (fewer slices than the plan's
+// measure of sum lengths asks for).
+template <int KW, bool FOLD>
 __global__ __launch_bounds__(NT * KW, KW == 1 ? 2 : 1) void tile_kernel(DevTensor t, const uint16_t* __restrict__ xh,
                                                                          uint32_t M, const int32_t* __restrict__ xe,
                                                                          void* __restrict__ y, uint32_t y_bf16,
@@ -414,7 +416,24 @@ __global__ __launch_bounds__(NT * KW, KW == 1 ? 2 : 1) void tile_kernel(DevTenso
   };
   using I0 = std::integral_constant<int, 0>;
   using I1 = std::integral_constant<int, 1>;
+  // FOLD: the first half's sums, fragment 3's in the output tile's LDS (each lane
+  // its own; 64 registers more than the loop's would not fit two waves per SIMD).
+  float16v half[3];
+  float* const half3 = reinterpret_cast<float*>(smem_all + out_offset<KW>()) + (threadIdx.x >> 6) * 1024u + lane;
+  static_assert(!FOLD || NT * KW * 16 * 4 <= BM * LDO * 2, "fragment 3 fits the output tile");
   uint32_t i = 0;
+  if constexpr (FOLD) {   // a loop of its own: a fold inside the one below copies the accumulators every round
+    for (; i < KT / 4 * 2; i += 2) {
+      body(i, I0{});
+      body(i + 1, I1{});
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) half3[64 * r] = acc[3][r];
+#pragma unroll
+    for (int f = 0; f < 3; ++f) half[f] = acc[f];
+#pragma unroll
+    for (int f = 0; f < 4; ++f) acc[f] = float16v{};
+  }
   for (; i + 2 < KT; i += 2) {
     body(i, I0{});
     body(i + 1, I1{});
@@ -430,6 +449,12 @@ __global__ __launch_bounds__(NT * KW, KW == 1 ? 2 : 1) void tile_kernel(DevTenso
       last(STAGE(1), bf[1]);
     else
       last(STAGE(0), bf[0]);
+  }
+  if constexpr (FOLD) {
+#pragma unroll
+    for (int f = 0; f < 3; ++f) acc[f] += half[f];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[3][r] += half3[64 * r];
   }
 #undef STAGE
 
@@ -727,6 +752,7 @@ __device__ __forceinline__ u32x4 res_operand(const uint32_t* s_res, ResWalk& w, 
 __device__ __forceinline__ void keep_here(const u32x4& v) { asm volatile("" ::"v"(v)); }
 
 // gridDim.x = tiles_m * tiles_n, gridDim.y = K slices of kt_per_split tiles.
+template <bool FOLD>
 __global__ __launch_bounds__(NT, 1) void tile_cb4_kernel(DevTensor t, const uint16_t* __restrict__ xh, uint32_t M,
                                                          const int32_t* __restrict__ xe, void* __restrict__ y,
                                                          uint32_t y_bf16, float* __restrict__ partial,
@@ -957,7 +983,19 @@ __global__ __launch_bounds__(NT, 1) void tile_cb4_kernel(DevTensor t, const uint
   };
   using I0 = std::integral_constant<int, 0>;
   using I1 = std::integral_constant<int, 1>;
+  float16v half[4];   // FOLD: the first half's sums (the lo plane's weigh 2^-11)
   uint32_t i = 0;
+  if constexpr (FOLD) {   // a loop of its own: a fold inside the one below copies the accumulators every round
+    for (; i < KT / 4 * 2; i += 2) {
+      body(i, I0{});
+      body(i + 1, I1{});
+    }
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+      half[f] = acc[f];
+      acc[f] = float16v{};
+    }
+  }
   for (; i + 2 < KT; i += 2) {
     body(i, I0{});
     body(i + 1, I1{});
@@ -967,6 +1005,10 @@ __global__ __launch_bounds__(NT, 1) void tile_cb4_kernel(DevTensor t, const uint
     ++i;
   }
   last(i, (i & 1) != 0);
+  if constexpr (FOLD) {
+#pragma unroll
+    for (int f = 0; f < 4; ++f) acc[f] += half[f];
+  }
 #undef STAGE
 
   // Epilogue: w * 2^e = hi + lo * 2^-11, so y = (acc + accl * 2^-11) * 2^-(e + xe).
@@ -1054,6 +1096,7 @@ __global__ __launch_bounds__(NT, 1) void tile_cb4_kernel(DevTensor t, const uint
 
 struct Plan {
   uint32_t tiles_m, tiles_n, kw, splits, kps;
+  bool fold;
   size_t xe_off, xh_off, partial_off, bytes;
 };
 
@@ -1066,8 +1109,11 @@ inline size_t al256(size_t v) { return (v + 255) & ~size_t(255); }
 // takes more than 4 slices.  Where one workgroup fills a CU the grid stays
 // within the 256 CUs: a slice more put 288 workgroups on them, two rounds of
 // two thirds (M = 200, 2048 -> 6144, 96 tiles, whole call: g64 32.8 -> 24.6 us, cb4 59.2 ->
-// 42.8).  The workspace is sized for the slice count rounded up, the most a
-// call of the shape has needed.
+// 42.8).  The slice count rounded up stays the measure of a sum's length: where the
+// grid has fewer slices, each is summed in two halves (fold; relative error of
+// 200 tokens 2048 -> 6144 on 3 slices / 2 whole / 2 in halves: g64 1.29 / 1.52 / 1.15e-7,
+// cb4 1.82 / 2.17 / 1.61e-7).  The workspace is sized for it as well, the most a call
+// of the shape has needed.
 constexpr size_t kMaxPartialBytes = (size_t)16 << 20;
 
 inline Plan plan(const DevTensor& t, uint32_t m) {
@@ -1092,6 +1138,7 @@ inline Plan plan(const DevTensor& t, uint32_t m) {
     p.kps = (ktt + splits - 1) / splits;
     p.splits = (ktt + p.kps - 1) / p.kps;
   }
+  p.fold = p.splits < reserve;
   // With more than 4 K slices each way would walk only a few tiles: one
   // K-way per workgroup is then faster (M = 128: 11.9 against 12.7 us at
   // 6144 x 2048, 12.8 against 14.2 us at 2048 x 6144).
@@ -1103,15 +1150,15 @@ inline Plan plan(const DevTensor& t, uint32_t m) {
   return p;
 }
 
-template <int KW>
+template <int KW, bool FOLD>
 hipError_t launch_tile(const DevTensor& t, const uint16_t* xh, uint32_t m, const int32_t* xe, void* y, bool y_bf16,
                        float* partial, const Plan& p, hipStream_t s) {
   constexpr size_t lds = lds_bytes<KW>();
   static_assert(lds <= 160 * 1024, "LDS budget");
-  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&tile_kernel<KW>),
+  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&tile_kernel<KW, FOLD>),
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (attr != hipSuccess) return attr;
-  hipLaunchKernelGGL((tile_kernel<KW>), dim3(p.tiles_m * p.tiles_n, p.splits), dim3(NT * KW), lds, s, t, xh, m, xe, y,
+  hipLaunchKernelGGL((tile_kernel<KW, FOLD>), dim3(p.tiles_m * p.tiles_n, p.splits), dim3(NT * KW), lds, s, t, xh, m, xe, y,
                      (uint32_t)y_bf16, partial, p.kps, p.tiles_m);
   return hipGetLastError();
 }
@@ -1135,6 +1182,7 @@ inline Plan plan_cb4(const DevTensor& t, uint32_t m) {
   splits = std::min(splits, std::max(1u, 256u / tiles));
   p.kps = (ktt + splits - 1) / splits;
   p.splits = (ktt + p.kps - 1) / p.kps;
+  p.fold = p.splits < reserve;
   p.xe_off = 0;
   p.xh_off = al256((size_t)m * 4);
   p.partial_off = p.xh_off + al256((size_t)m * t.kp * 2);
@@ -1142,12 +1190,13 @@ inline Plan plan_cb4(const DevTensor& t, uint32_t m) {
   return p;
 }
 
+template <bool FOLD>
 inline hipError_t launch_tile_cb4(const DevTensor& t, const uint16_t* xh, uint32_t m, const int32_t* xe, void* y,
                                   bool y_bf16, float* partial, const Plan& p, hipStream_t s) {
-  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&tile_cb4_kernel),
+  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&tile_cb4_kernel<FOLD>),
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)kC4Bytes);
   if (attr != hipSuccess) return attr;
-  hipLaunchKernelGGL(tile_cb4_kernel, dim3(p.tiles_m * p.tiles_n, p.splits), dim3(NT), kC4Bytes, s, t, xh, m, xe, y,
+  hipLaunchKernelGGL(tile_cb4_kernel<FOLD>, dim3(p.tiles_m * p.tiles_n, p.splits), dim3(NT), kC4Bytes, s, t, xh, m, xe, y,
                      (uint32_t)y_bf16, partial, p.kps, p.tiles_m);
   return hipGetLastError();
 }
@@ -1190,8 +1239,10 @@ hipError_t launch_gemm_tile(const DevTensor& t, const uint16_t* x, uint32_t m, v
   float* partial = reinterpret_cast<float*>(base + p.partial_off);
   hipError_t e = gt::launch_xprep(x, m, t.cols, t.kp, xh, xe, s);
   if (e != hipSuccess) return e;
-  e = p.kw == 1 ? gt::launch_tile<1>(t, xh, m, xe, y, y_bf16, partial, p, s)
-                : gt::launch_tile<2>(t, xh, m, xe, y, y_bf16, partial, p, s);
+  // (fold comes with two K-ways: the slice count is lowered for those only)
+  e = p.kw == 1 ? gt::launch_tile<1, false>(t, xh, m, xe, y, y_bf16, partial, p, s)
+      : p.fold  ? gt::launch_tile<2, true>(t, xh, m, xe, y, y_bf16, partial, p, s)
+                : gt::launch_tile<2, false>(t, xh, m, xe, y, y_bf16, partial, p, s);
   if (e != hipSuccess || p.splits == 1) return e;
   return launch_gemm_reduce(partial, p.splits, nullptr, xe, m, t.rows, y, y_bf16, s);
 }
@@ -1213,7 +1264,8 @@ hipError_t launch_gemm_tile_cb4(const DevTensor& t, const uint16_t* x, uint32_t 
   float* partial = reinterpret_cast<float*>(base + p.partial_off);
   hipError_t e = gt::launch_xprep(x, m, t.cols, t.kp, xh, xe, s);
   if (e != hipSuccess) return e;
-  e = gt::launch_tile_cb4(t, xh, m, xe, y, y_bf16, partial, p, s);
+  e = p.fold ? gt::launch_tile_cb4<true>(t, xh, m, xe, y, y_bf16, partial, p, s)
+             : gt::launch_tile_cb4<false>(t, xh, m, xe, y, y_bf16, partial, p, s);
   if (e != hipSuccess || p.splits == 1) return e;
   return launch_gemm_reduce(partial, p.splits, nullptr, xe, m, t.rows, y, y_bf16, s);
 }
