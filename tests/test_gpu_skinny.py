@@ -162,3 +162,34 @@ def test_skinny_small_centroids(eng):
     want = np.ldexp(X.astype(np.float64) @ W.T, -118)
     rel = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
     assert rel.max() <= 4 * 2.0 ** -24, rel      # the sums' own error is 0.7 .. 0.9e-7; lost centroid bits gave 2^-15
+
+
+@pytest.mark.parametrize("kind", ["cb4", "g64", "q8", "q4_0"])
+@pytest.mark.parametrize("rows,cols,M", [
+    (40, 600, 4), (2048, 1300, 3), (2049, 2600, 4), (40, 1500, 7), (40, 5000, 6), (70, 8200, 11), (4200, 3100, 16),
+    (33, 12300, 9)])
+def test_skinny_f32_forms(eng, kind, rows, cols, M):
+    """f32 activations: half tiles of one and of several phases up to 2048 rows,
+    and K ranges of one to several thousand columns above 8 tokens, plain and
+    gated (silu(g) u: |silu'| <= 1.1)."""
+    print(f"skinny f32 forms {kind} rows={rows} cols={cols} M={M}", flush=True)
+    rows += rows & 1
+    m = synth.make_q40(rows, cols, seed=6) if kind == "q4_0" else make(kind, rows, cols, seed=6)
+    t = eng.upload_packed(m)
+    X = (np.random.default_rng(cols).standard_normal((M, cols)) / cols ** 0.5).astype(np.float32)
+    got = run_dev(eng, t, X, engine.DTYPE_F32, M, engine.DTYPE_F32)
+    F = rows // 2
+    xd, yd = eng.to_device(X), eng.alloc(M * F * 4)
+    eng.ffn_glu_dev(t, xd.ptr, engine.DTYPE_F32, M, yd.ptr, engine.DTYPE_F32, F, engine.ACT_SILU, eng.stream)
+    eng.synchronize()
+    act = yd.download(np.float32, (M, F))
+    for b in (xd, yd, t):
+        b.free()
+    W = oracle.decode_rows(m).astype(np.float64)
+    want = X.astype(np.float64) @ W.T
+    bound = (160 + cols / 128) * 2.0 ** -24 * (np.abs(X) @ np.abs(W).T)
+    assert np.all(np.abs(got - want) <= bound)
+    g, u = want[:, :F], want[:, F:]
+    s = g / (1 + np.exp(-g))
+    tol = 1.1 * bound[:, :F] * np.abs(u) + np.abs(s) * bound[:, F:] + 2.0 ** -20 * np.abs(s * u) + 1e-12
+    assert np.all(np.abs(act - s * u) <= tol)

@@ -1,5 +1,7 @@
 // gemm_skinny.hip -- entry to the few-token MFMA kernels (gemm_skinny_impl.hpp),
 // instantiated by weight kind in gemm_skinny_{cb4,g64,q40,q8}.hip.
+#include <algorithm>
+
 #include "common.hpp"
 
 namespace vxt {
@@ -31,15 +33,31 @@ static SkinnyArgs args(const DevTensor& t, const void* x, bool x_bf16, uint32_t 
   a.x_vec = reinterpret_cast<uintptr_t>(x) % 16 == 0 && t.cols % 8 == 0 && ((size_t)t.cols * esz) % 16 == 0;
   a.y_bf16 = y_bf16;
   a.skip_zero = m <= 8;   // batch_m 1..8 is the GEMV, above the GEMM
-  a.kslice = (t.cols + 1023u) / 1024u * 1024u;
+  a.kslice = (t.cols + 1023u) / 1024u * 1024u;   // one range
   return a;
 }
 
 // K ranges of a call, each a set of workgroups of its own, summed by the
-// split-K reduction.
-static uint32_t k_slices(const DevTensor& t, uint32_t m, bool x_bf16) {
-  if (!x_bf16 || m <= 8) return 1;
-  return (t.cols + 2047u) / 2048u;
+// split-K reduction; their columns (a multiple of 1024) in `cols`.  bf16
+// activations above 8 tokens: 2048 columns.  f32 ones past 2048 columns: a
+// workgroup fills a CU and takes some 3 us per 1024 columns, so the fewest ranges
+// that cut rounds over the 256 CUs x columns by a sixth or more (16 tokens, us,
+// one range and the two-phase path against this: cb4 8192 -> 2048 52 / 43 against
+// 28.6, Q4_0 8192 -> 1024 42 / 32 against 14.6, g64 6144 -> 2048 35 / 26 against 14.6,
+// Q8_0 12288 -> 512 42 / 31 against 10.8).
+static uint32_t k_slices(const DevTensor& t, uint32_t m, bool x_bf16, uint32_t* cols = nullptr) {
+  const uint32_t kt = (t.cols + 1023u) / 1024u;
+  uint32_t per = kt;
+  if (m > 8 && x_bf16) {
+    per = 2;
+  } else if (m > 8 && kt > 2) {
+    const uint32_t tr = t.kind == KIND_G64 ? 32u : 16u, tiles = (t.rows + tr - 1u) / tr;   // rows of a workgroup
+    auto cost = [&](uint32_t p) { return (tiles * ((kt + p - 1u) / p) + 255u) / 256u * p; };
+    for (uint32_t p = kt - 1u; p > 0; --p)
+      if (cost(p) * 6u <= cost(per) * 5u) per = p;
+  }
+  if (cols) *cols = per * 1024u;
+  return (kt + per - 1u) / per;
 }
 
 // The most tokens of one call.
@@ -52,9 +70,10 @@ size_t skinny_workspace_bytes(const DevTensor& t, uint32_t m, bool x_bf16) {
 
 hipError_t launch_skinny(const DevTensor& t, const void* x, bool x_bf16, uint32_t m, void* y, bool y_bf16, void* ws,
                          hipStream_t s) {
-  const uint32_t sl = k_slices(t, m, x_bf16);
+  uint32_t per;
+  const uint32_t sl = k_slices(t, m, x_bf16, &per);
   SkinnyArgs a = args(t, x, x_bf16, m, sl > 1 ? ws : y, sl > 1 ? false : y_bf16);
-  if (sl > 1) a.kslice = 2048;
+  if (sl > 1) a.kslice = per;
   const hipError_t e = launch_any(t, a, x_bf16, s);
   if (e != hipSuccess || sl == 1) return e;
   return launch_gemm_reduce(static_cast<const float*>(ws), sl, nullptr, nullptr, m, t.rows, y, y_bf16, s);
@@ -71,7 +90,7 @@ hipError_t launch_skinny(const DevTensor& t, const void* x, bool x_bf16, uint32_
 bool skinny_glu_takes(const DevTensor& t, const void* x, uint32_t m, bool x_bf16, int mode) {
   if (m <= 8) return t.kind != KIND_Q8 || m == 2 || !args(t, x, x_bf16, m, nullptr, false).x_vec || !x_bf16;
   if (mode != kGemmAuto && mode != kGemmAutoOwn) return false;
-  if (m <= 16) return true;
+  if (m <= 16) return x_bf16 || k_slices(t, m, x_bf16) == 1;   // f32: where the plain form needs no K ranges
   const size_t w = (size_t)t.cols * t.rows, M1 = 1000 * 1000;
   return m <= skinny_max_m(x_bf16) && t.cols <= 2048 && w <= (m <= 32 ? 34 : 26) * M1;
 }

@@ -102,6 +102,7 @@ constexpr int kWaves = 8;
 constexpr int kThreads = 64 * kWaves;
 constexpr uint32_t kStreamRows = 32768;
 constexpr uint32_t kHalfRows = 4096;
+constexpr uint32_t kHalfRowsF32 = 2048;   // one workgroup per CU: one round
 
 // f32 as three bf16 terms, each the high half of a word (what the low halves
 // hold is not read): v = h + m 2^-8 + l 2^-16 exactly, subnormals too.  Inf and
@@ -987,9 +988,20 @@ hipError_t launch_plain(const DevTensor& t, const Args& a, bool x_bf16, hipStrea
   constexpr bool G = KIND == KIND_G64;
   const uint32_t K = t.cols, M = a.M, n = t.rows;
   if (!x_bf16) {
-    if (M <= 4)
+    // Half tiles: one round of 256 workgroups at most, and a K whose phases they
+    // halve (4 tokens, us: cb4 4096 -> 1024 13.3 -> 9.0, 8192 -> 1024 27.6 -> 18.1, g64
+    // 4096 -> 1024 9.0 -> 6.5; 8 tokens Q8_0 4096 -> 1024 12.1 -> 8.0; from 2049 rows on,
+    // two rounds, 4 tokens of cb4 3072 -> 4096 12.4 against 16.1).
+    const bool half = n <= kHalfRowsF32 && K > (G ? 2048u : M <= 4 ? 512u : 1024u);
+    if constexpr (!G) {
+      if (M <= 4 && half && K <= 2048) return launch<KIND, 3, 1, 4, 1, 1, false, false, true>(t, a, n, s);
+      if (M > 4 && M <= 8 && half) return launch<KIND, 3, 1, 8, 1, 1, true, false, true>(t, a, n, s);
+    }
+    if (M <= 4) {
+      if (half) return launch<KIND, 3, 1, 4, 1, 1, true, false, true>(t, a, n, s);
       return K <= 2048 ? launch<KIND, 3, 1, 4, 1, N1, false, false>(t, a, n, s)
                        : launch<KIND, 3, 1, 4, 1, N1, true, false>(t, a, n, s);
+    }
     return launch<KIND, 3, 1, 16, G ? 2 : 1, 1, true, false>(t, a, n, s);   // 1024 columns: four g64 chunks
   }
   if (n >= kStreamRows && K <= 2048 && M <= 16) {
@@ -1031,9 +1043,14 @@ hipError_t launch_glu(const DevTensor& t, const Args& a, bool x_bf16, hipStream_
   constexpr int N1 = 256 / kChunk<KIND>;
   constexpr bool G = KIND == KIND_G64;
   const uint32_t K = t.cols, M = a.M, n = a.y_stride;
-  if (!x_bf16)
+  if (!x_bf16) {
+    const bool half = t.rows <= kHalfRowsF32 && K > (G ? 2048u : M <= 4 ? 512u : 1024u);   // as the plain form
+    if (M <= 4 && half) return launch<KIND, 3, 1, 4, 1, 1, true, true, true>(t, a, n, s);
+    if constexpr (!G)
+      if (M <= 8 && half) return launch<KIND, 3, 1, 8, 1, 1, true, true, true>(t, a, n, s);
     return M <= 4 ? launch<KIND, 3, 1, 4, 1, N1, true, true>(t, a, n, s)
                   : launch<KIND, 3, 1, 16, G ? 2 : 1, 1, true, true>(t, a, n, s);
+  }
   // Half tiles for the sizes where the plain form takes them: the sums are
   // those of the plain form, bit for bit (up to 8 tokens).
   if (M <= 8 && t.rows <= kHalfRows && (!G || K > 2048)) {
