@@ -193,3 +193,18 @@ def test_skinny_f32_forms(eng, kind, rows, cols, M):
     s = g / (1 + np.exp(-g))
     tol = 1.1 * bound[:, :F] * np.abs(u) + np.abs(s) * bound[:, F:] + 2.0 ** -20 * np.abs(s * u) + 1e-12
     assert np.all(np.abs(act - s * u) <= tol)
+
+
+@pytest.mark.parametrize("rows,cols,M", [(8192, 2050, 11), (8201, 4097, 16), (12288, 2304, 12)])
+def test_g64_all_of_k_in_one_range(eng, rows, cols, M):
+    """g64 from 11 tokens and 8192 rows: all of K in several phases of one
+    workgroup, the last one ragged; the file's bound."""
+    print(f"g64 one range rows={rows} cols={cols} M={M}", flush=True)
+    m = make("g64", rows, cols, seed=2)
+    t = eng.upload_packed(m)
+    xh = f32_to_bf16_bits(np.random.default_rng(M).standard_normal((M, cols)).astype(np.float32))
+    X = bf16_bits_to_f32(xh).reshape(M, cols).astype(np.float64)
+    got = run_dev(eng, t, xh, engine.DTYPE_BF16, M, engine.DTYPE_F32)
+    t.free()
+    W = oracle.decode_rows(m).astype(np.float64)
+    assert np.all(np.abs(got - X @ W.T) <= (160 + cols / 128) * 2.0 ** -24 * (np.abs(X) @ np.abs(W).T))

@@ -1255,26 +1255,36 @@ static size_t path_workspace_bytes(Path path, const DevTensor& t, uint32_t m, bo
 }
 
 // The few-token kernels (gemm_skinny.hip) take a call in AUTO up to 16 tokens
-// (within the workspace rule of takes_skinny), and up to 32 and 64 while each weight's decode, repeated for every
-// 32 tokens, is cheaper than a panel, as measured by kind (whole call, us,
-// this against the general path; K -> N):
+// (within the workspace rule of takes_skinny), and up to 32 and 64 while each
+// weight's decode, repeated for every 32 tokens, is cheaper than a panel, as
+// measured by kind (whole call, us, this against the general path; K -> N):
 //   M = 17..32: cb4, Q4_0 always (32 tokens 2048 -> 6144 15.7 / 11.6 against
 //   36.0 / 29.7, 2048 -> 151936 238 / 194 against 858 / 526); g64 and Q8_0 up
-//   to 34 M weights, Q8_0 also K <= 4096 (g64 / Q8_0 2048 -> 16384 19.1 / 17.5
-//   against 21.2 / 19.0; 8192 -> 4096 23.2 / 22.3 against 23.4 / 19.0;
-//   2048 -> 151936 170 / 156 against 116 / 142);
+//   to 34 M weights with K <= 2048 (2048 -> 16384 19.1 / 17.5 against 21.2 / 19.0;
+//   2048 -> 151936 170 / 156 against 116 / 142), above g64 up to 26 M, with K =
+//   3073 .. 6144 up to 17 M (17 tokens 8192 -> 2048 12.3 against 16.5; 4096 -> 6144 and
+//   6144 -> 4096 1.10 and 1.13 times as long), and Q8_0 not (17 tokens 4096 -> 1024 10.5
+//   against 8.9);
 //   M = 33..64: cb4 up to 34 M weights and K <= 4096 (2048 -> 16384 52 against
 //   66; 6144 -> 2048 40 against 36), Q4_0 up to 24 M (4096 -> 4096 24 against
 //   35; 8192 -> 4096 46 against 39), g64 up to 13 M (6144 -> 2048 21.7 against
 //   23.1; 2048 -> 16384 38 against 28), Q8_0 up to 8 M (2048 -> 2048 8.9 against
 //   11.7; 4096 -> 4096 20.4 against 19.1).
+// g64 also leaves them with bf16 activations and many rows, where the fused kernel
+// decodes a table once for more tokens: from 11 tokens with K > 2048 (16 tokens
+// 3072 -> 16384 1.28, 4096 -> 32768 70 against 50.7) or K < 1024 (512 -> 16384 1.21
+// times as long; 2048 -> 16384 0.90; from 17 tokens past 24576 rows), from 33 with K <=
+// 2048 (512 -> 16384 16.8 against 14.5; 12288 rows level).
 bool skinny_takes(const DevTensor& t, uint32_t m, bool x_bf16) {
+  const size_t w = (size_t)t.cols * t.rows, M1 = 1000 * 1000;
+  if (t.kind == KIND_G64 && x_bf16 && t.rows > 12288u && m > 10 &&
+      (t.cols > 2048u || m > 32 || (t.cols < 1024u && t.rows < 32768u && (m <= 16 || t.rows > 24576u))))
+    return false;
   if (m <= 16) return true;
   if (m > skinny_max_m(x_bf16)) return false;
-  const size_t w = (size_t)t.cols * t.rows, M1 = 1000 * 1000;
   if (m <= 32) {
-    if (t.kind == KIND_Q8) return w <= 34 * M1 && t.cols <= 4096;
-    return t.kind != KIND_G64 || w <= 34 * M1;
+    if (t.kind == KIND_Q8) return w <= 34 * M1 && t.cols <= 2048;
+    return t.kind != KIND_G64 || w <= (t.cols <= 2048 ? 34 : t.cols > 3072 && t.cols <= 6144 ? 17 : 26) * M1;
   }
   switch (t.kind) {
     case KIND_CB4: return w <= 34 * M1 && t.cols <= 4096;
@@ -1297,10 +1307,12 @@ size_t gemm_workspace_bytes(const DevTensor& t, uint32_t m, bool x_bf16, int mod
 }
 
 // The few-token kernels' K ranges can need more than that (g64 and Q8_0, whose
-// fused kernel may have no partial sums: 16 tokens at K = 2112 .. 4096 from
-// 32768 rows, 8192 from 12288): such a call keeps the general path.  The choice
-// looks at what the call reserves, not at what the workspace has grown to, so a
-// call's kernel, and its bits, do not depend on the calls before it.
+// fused kernel may have few partial sums or none: up to 16 tokens at K = 2112 ..
+// 4096 from 32768 rows, 6144 from 16384, 8192 from 12288): such a call keeps the general
+// path (12 tokens Q8_0 8192 -> 12288 51.5 us against 35.7; in ranges made longer until they
+// fit 55.7).  The choice looks at what the call reserves, not at what the
+// workspace has grown to, so a call's kernel, and its bits, do not depend on the
+// calls before it, and a capture needs no more than it did.
 static bool takes_skinny(const DevTensor& t, uint32_t m, bool x_bf16, int mode) {
   return (mode == kGemmAuto || mode == kGemmAutoOwn) && skinny_takes(t, m, x_bf16) &&
          skinny_workspace_bytes(t, m, x_bf16) <= gemm_workspace_bytes(t, m, x_bf16, mode);

@@ -39,17 +39,19 @@ static SkinnyArgs args(const DevTensor& t, const void* x, bool x_bf16, uint32_t 
 
 // K ranges of a call, each a set of workgroups of its own, summed by the
 // split-K reduction; their columns (a multiple of 1024) in `cols`.  bf16
-// activations above 8 tokens: 2048 columns.  f32 ones past 2048 columns: a
-// workgroup fills a CU and takes some 3 us per 1024 columns, so the fewest ranges
-// that cut rounds over the 256 CUs x columns by a sixth or more (16 tokens, us,
-// one range and the two-phase path against this: cb4 8192 -> 2048 52 / 43 against
+// activations above 8 tokens: 2048 columns, but all of K for g64 from 11 tokens and
+// 8192 rows (16 tokens 2304 -> 12288 the sliced form takes 1.14 times as long, the
+// fused kernel 0.95 times; cb4, Q8_0, Q4_0 in one range 1.1 .. 1.6 times as long).
+// f32 ones past 2048 columns: a workgroup fills a CU and takes some 3 us per 1024
+// columns, so the fewest ranges that cut rounds over the 256 CUs x columns by a
+// sixth or more (16 tokens, us, one range and the two-phase path against this: cb4 8192 -> 2048 52 / 43 against
 // 28.6, Q4_0 8192 -> 1024 42 / 32 against 14.6, g64 6144 -> 2048 35 / 26 against 14.6,
 // Q8_0 12288 -> 512 42 / 31 against 10.8).
 static uint32_t k_slices(const DevTensor& t, uint32_t m, bool x_bf16, uint32_t* cols = nullptr) {
   const uint32_t kt = (t.cols + 1023u) / 1024u;
   uint32_t per = kt;
   if (m > 8 && x_bf16) {
-    per = 2;
+    if (!(t.kind == KIND_G64 && m > 10 && m <= 16 && t.rows >= 8192u)) per = 2;
   } else if (m > 8 && kt > 2) {
     const uint32_t tr = t.kind == KIND_G64 ? 32u : 16u, tiles = (t.rows + tr - 1u) / tr;   // rows of a workgroup
     auto cost = [&](uint32_t p) { return (tiles * ((kt + p - 1u) / p) + 255u) / 256u * p; };
@@ -81,16 +83,27 @@ hipError_t launch_skinny(const DevTensor& t, const void* x, bool x_bf16, uint32_
 
 // Whether a gated call takes the fused form: up to 8 tokens always (but Q8_0
 // with 3 .. 8 aligned bf16 tokens, whose plain GEMV has kernels of its own: the
-// staged form keeps its sums), above (in AUTO) up to 16, and up to 64 bf16 tokens while K fits one phase range and
-// the decode, repeated for every 32 tokens, stays below the staged form's
-// GEMM, f32 gate and up rows and element-wise pass (32 / 64 tokens, K = 2048,
-// n_ff = 6144, us against the staged form: cb4 27 / 40 against 58 / 59, g64 20
-// / 29 against 25 / 34, Q4_0 22 / 32 against 41 / 40, Q8_0 18 / 26 against 23
-// / 30).
+// staged form keeps its sums), above (in AUTO) up to 16, and up to 64 bf16 tokens
+// while K fits one phase range and the decode, repeated for every 32 tokens, stays
+// below the staged form's GEMM, f32 gate and up rows and element-wise pass (32 / 64
+// tokens, K = 2048, n_ff = 6144, us against the staged form: cb4 27 / 40 against 58
+// / 59, g64 20 / 29 against 25 / 34, Q4_0 22 / 32 against 41 / 40, Q8_0 18 / 26
+// against 23 / 30).  f32 activations: where the plain form needs no K ranges.  g64
+// leaves with many rows where its staged GEMM is the fused kernel and ahead
+// (fused form over staged: 16 tokens n_ff = 11008, K = 512 1.50, 3072 1.13, 8192 1.16;
+// 33 tokens 512 1.37; 17 tokens n_ff = 14336, 512 1.23), Q8_0 so above 32 tokens (33
+// tokens 512, n_ff = 11008 1.56) and with few rows of a long K (16 tokens 8192,
+// n_ff = 64 .. 1024 1.25; 1536 0.75).
 bool skinny_glu_takes(const DevTensor& t, const void* x, uint32_t m, bool x_bf16, int mode) {
   if (m <= 8) return t.kind != KIND_Q8 || m == 2 || !args(t, x, x_bf16, m, nullptr, false).x_vec || !x_bf16;
   if (mode != kGemmAuto && mode != kGemmAutoOwn) return false;
-  if (m <= 16) return x_bf16 || k_slices(t, m, x_bf16) == 1;   // f32: where the plain form needs no K ranges
+  const uint32_t n_ff = t.rows / 2;
+  if (x_bf16 && t.kind == KIND_G64 && m > 10) {
+    if (t.cols < 1024 && n_ff > (m > 16 && m <= 32 ? 12288u : 8192u)) return false;
+    if (t.cols > 2048 && n_ff >= 8192) return false;
+  }
+  if (x_bf16 && t.kind == KIND_Q8 && (m > 32 ? t.cols < 1024 && n_ff > 8192 : t.cols > 6144 && n_ff < 1536)) return false;
+  if (m <= 16) return x_bf16 || k_slices(t, m, x_bf16) == 1;
   const size_t w = (size_t)t.cols * t.rows, M1 = 1000 * 1000;
   return m <= skinny_max_m(x_bf16) && t.cols <= 2048 && w <= (m <= 32 ? 34 : 26) * M1;
 }

@@ -1033,8 +1033,10 @@ hipError_t launch_plain(const DevTensor& t, const Args& a, bool x_bf16, hipStrea
     if (K <= 4096) return launch<KIND, 1, 1, 8, 1, 2 * N1, false, false>(t, a, n, s);
     return launch<KIND, 1, 1, 8, 1, 2 * N1, true, false>(t, a, n, s);
   }
-  // More tokens: K ranges of at most 2048 columns (gemm_skinny.hip sums them)
-  if (M <= 16) return launch<KIND, 1, 1, 16, 1, N1, false, false>(t, a, n, s);
+  // More tokens: K ranges of at most 2048 columns (gemm_skinny.hip sums them), or one of several phases
+  if (M <= 16)
+    return std::min(K, a.kslice) <= 2048 ? launch<KIND, 1, 1, 16, 1, N1, false, false>(t, a, n, s)
+                                         : launch<KIND, 1, 1, 16, 1, N1, true, false>(t, a, n, s);
   return launch<KIND, 1, 2, 32, 2, N1, true, false>(t, a, n, s);
 }
 
