@@ -904,17 +904,32 @@ inline Plan plan(const DevTensor& t, uint32_t m, bool x_bf16, bool lib) {
   // 35.6 / 30.2 / 33.8 (41.0 / 33.3 / 39.0); 300, 2048 -> 6144 60.4 / 42.8 / 55.6
   // (90.3 / 67.5 / 86.8; 64.5 / 44.5 / 60.1 on 128 x 128); 2048, 2048 -> 2048 71.3 /
   // 55.7 / 67.9 (96.0 / 76.8 / 92.8).  Up to 128 tokens, and below 32 tiles (64 up to
-  // 191 tokens), the other's 64-row tiles fill more of the chip.
-  if (!x_bf16 && !lib && m > 128 && t128 >= (m >= 192 ? 32u : 64u) && fits) {
+  // 191 tokens), the other's 64-row tiles fill more of the chip; up to 255 tokens
+  // also with K < 1024 (191 tokens 512 -> 6144 30.6 / 21.3 / 28.9 against 26.3 / 17.6 /
+  // 24.8; g64 up to 128 tiles of K = 1024: 1024 -> 4096 27.5 against 23.5), up to 191 where two MFMAs more per product make the empty rows of 128-row
+  // tiles dear (hi/lo panels of 128 M weights: 130 tokens 8192 -> 16384 cb4 526 against
+  // 472, Q8 444 against 402, Q4_0 466 against 419; g64 233 against 296).
+  const size_t weights = (size_t)t.cols * t.rows;
+  const bool deep = m >= 256 || (t.cols >= 1024 && !(t.kind == KIND_G64 && t.cols == 1024 && t128 <= 128) && !(m < 192 && pl.wmode != kWPlain && weights >= (size_t)128000000));
+  if (!x_bf16 && !lib && m > 128 && t128 >= (m >= 192 ? 32u : 64u) && deep && fits) {
     pl.d3mode = pl.wmode == kWPlain ? 0 : 1;
     pl.d3cfg = ((m + 255) / 256) * ((t.rows + 127) / 128) * pl.splits >= 192 ? 4 : 3;
   }
   // bf16 below 96 tiles: up to 255 tokens the register-staged kernel has 64 x 64
   // tiles, which read each operand twice as often; this one is ahead from 48 tiles,
   // with K >= 4096 from 32 (Q4_0, whole call: 72 tokens 2048 -> 6144 34.8 -> 31.6 us,
-  // 200 36.3 -> 29.9, 70 of 4096 -> 8192 49.4 -> 43.5).
+  // 200 36.3 -> 29.9, 70 of 4096 -> 8192 49.4 -> 43.5).  Not above 128 tokens with
+  // K <= 1024 (Q8_0 255 tokens 512 / 1024 -> 4096 19.4 / 27.5 against 15.5 / 23.8), not up to
+  // 64 tokens with K >= 8192, cb4 6144 (half of a tile empty: Q4_0 8192 -> 4096 / 6144
+  // 43.3 / 60 against 38.7 / 49, cb4 6144 -> 4096 58.8 against 51.6), not past 60 M weights
+  // of cb4 (96 tokens 8192 -> 8192 194 against 181), 80 M with K > 8192 else (Q4_0
+  // 12288 -> 8192 182 against 161).
   const bool few = t128 < 96;
-  if (x_bf16 && !lib && fits && (!few || (m < 256 && (t128 >= 48 || (t128 >= 32 && ktiles >= 64))))) {
+  const bool few_ok = m < 256 && (t128 >= 48 || (t128 >= 32 && ktiles >= 64)) && (m <= 128 || t.cols > 1024) &&
+                      (m > 64 || t.cols < (t.kind == KIND_CB4 ? 6144u : 8192u)) &&
+                      (t.kind == KIND_CB4 ? weights <= (size_t)60000000
+                                          : t.cols <= 8192 || weights <= (size_t)80000000);
+  if (x_bf16 && !lib && fits && (!few || few_ok)) {
     pl.d3mode = pl.wmode == kWPlain ? 0 : pl.wmode == kWHiLo ? 1 : 2;
     const uint32_t m256 = (m + 255) / 256, t256 = m256 * ((t.rows + 127) / 128);
     if (pl.wmode == kWPlain && t.rows % 192 == 0 && m256 * (t.rows / 192) >= 192)
@@ -1189,7 +1204,8 @@ hipError_t launch_gemm_tile_cb4(const DevTensor& t, const uint16_t* x, uint32_t 
 // comparison.  Measured on MI355X (whole call, graph of 100 calls, TFLOP/s,
 // K x N = 2048 x 6144 / 6144 x 2048):
 //   g64 M = 64: fused 73 / 61, two-phase 68 / 61; M = 72: tile 95, two-phase
-//   78 (2048 x 6144); M = 100: tile 214, two-phase 161 (2048 x 12288); M = 128:
+//   78 (2048 x 6144); M = 100: tile 214, two-phase 161 (2048 x 12288; 16384 x
+//   512 34.3 against 27.7 us); M = 128:
 //   tile 134 / 118, two-phase 115 / 107; M = 512:
 //   tile 407 / 350, two-phase 300 / 325; with the two-phase planes in 1 KB
 //   pieces: M = 512: tile 409 / 358, two-phase 418 / 321; M = 768: tile
@@ -1229,7 +1245,9 @@ static Path general_path(const DevTensor& t, uint32_t m, bool x_bf16, int mode) 
     return Path::TileCb4;
   if (t.kind == KIND_G64 && x_bf16) {
     if (fused_ok && m <= kG64FusedMaxM) return Path::Fused;
-    if (tile_ok && m > kG64FusedMaxM && m < (t.cols > t.rows ? kTileMaxMTall : kTileMaxM)) return Path::Tile;
+    // (a few tiles of a very long K: the panel's rows fill more of the chip)
+    const bool narrow = m < 128 && t.cols > 8192 && t.cols / 16 >= t.rows;
+    if (tile_ok && m > kG64FusedMaxM && !narrow && m < (t.cols > t.rows ? kTileMaxMTall : kTileMaxM)) return Path::Tile;
     return Path::Panel;
   }
   if (fused_ok && (m <= kFusedMaxM || (t.kind == KIND_Q8 && t.cols >= t.rows && m < kQ8FusedMaxMTall)))
