@@ -1278,10 +1278,10 @@ static size_t path_workspace_bytes(Path path, const DevTensor& t, uint32_t m, bo
 // measured by kind (whole call, us, this against the general path; K -> N):
 //   M = 17..32: cb4, Q4_0 always (32 tokens 2048 -> 6144 15.7 / 11.6 against
 //   36.0 / 29.7, 2048 -> 151936 238 / 194 against 858 / 526); g64 and Q8_0 up
-//   to 34 M weights with K <= 2048 (2048 -> 16384 19.1 / 17.5 against 21.2 / 19.0;
-//   2048 -> 151936 170 / 156 against 116 / 142), above g64 up to 26 M, with K =
-//   3073 .. 6144 up to 17 M (17 tokens 8192 -> 2048 12.3 against 16.5; 4096 -> 6144 and
-//   6144 -> 4096 1.10 and 1.13 times as long), and Q8_0 not (17 tokens 4096 -> 1024 10.5
+//   to 34 M weights (2048 -> 16384 19.1 / 17.5 against 21.2 / 19.0; g64 8192 -> 4096
+//   22.7 against 24.3; 2048 -> 151936 170 / 156 against 116 / 142), g64 with K = 3073 ..
+//   6144 up to 17 M (17 tokens 4096 -> 4096 12.5 against 14.9; 4096 -> 6144 and 6144 ->
+//   4096 1.10 and 1.13 times as long), Q8_0 with K <= 2048 (17 tokens 4096 -> 1024 10.5
 //   against 8.9);
 //   M = 33..64: cb4 up to 34 M weights and K <= 4096 (2048 -> 16384 52 against
 //   66; 6144 -> 2048 40 against 36), Q4_0 up to 24 M (4096 -> 4096 24 against
@@ -1302,7 +1302,7 @@ bool skinny_takes(const DevTensor& t, uint32_t m, bool x_bf16) {
   if (m > skinny_max_m(x_bf16)) return false;
   if (m <= 32) {
     if (t.kind == KIND_Q8) return w <= 34 * M1 && t.cols <= 2048;
-    return t.kind != KIND_G64 || w <= (t.cols <= 2048 ? 34 : t.cols > 3072 && t.cols <= 6144 ? 17 : 26) * M1;
+    return t.kind != KIND_G64 || w <= (t.cols > 3072 && t.cols <= 6144 ? 17 : 34) * M1;
   }
   switch (t.kind) {
     case KIND_CB4: return w <= 34 * M1 && t.cols <= 4096;
