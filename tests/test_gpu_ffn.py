@@ -134,6 +134,41 @@ def test_gated_epilogue_matches_plain_gemv(eng, kind, M):
     t.free()
 
 
+# Two tokens around the limits where the generic kernel takes them (K = 1024,
+# 2048, 4096 and 6144, rows by kind), with ragged rows, K not a multiple of a
+# chunk and an odd K (no wide loads), against 64-bit sums.
+@pytest.mark.parametrize("kind", ["cb4", "g64", "q8", "q4_0"])
+@pytest.mark.parametrize("n_ff,cols", [(1, 1025), (301, 1031), (1024, 2048), (1025, 2000), (3, 2049), (1030, 2056),
+                                       (1100, 4104), (2049, 6144), (37, 6145), (1537, 6200)])
+def test_two_tokens(eng, kind, n_ff, cols):
+    gate, up, t = upload_gate_up(eng, kind, n_ff, cols, seed=n_ff + cols)
+    X = bf16_bits_to_f32(f32_to_bf16_bits(np.random.default_rng(cols).standard_normal((2, cols)).astype(np.float32)))
+    W = np.concatenate([oracle.decode_rows(gate), oracle.decode_rows(up)]).astype(np.float64)
+    want = X.astype(np.float64) @ W.T
+    # roundings of an f32 sum of K products in either kernel's order: at most
+    # this many half ulp of the sum of the products' magnitudes
+    bound = (160 + cols / 64) * 2.0 ** -24 * (np.abs(X).astype(np.float64) @ np.abs(W).T) + 1e-38
+    xd, yd = eng.to_device(f32_to_bf16_bits(X)), eng.alloc(4 * n_ff * 4)
+    eng.matmul_dev(t, xd.ptr, engine.DTYPE_BF16, 2, yd.ptr, engine.DTYPE_F32, eng.stream)
+    eng.synchronize()
+    got = yd.download(np.float32, (2, 2 * n_ff))
+    xd.free()
+    yd.free()
+    assert np.all(np.abs(got - want) <= bound)
+    g, u, bg, bu = want[:, :n_ff], want[:, n_ff:], bound[:, :n_ff], bound[:, n_ff:]
+    for activation in (engine.ACT_SILU, engine.ACT_GELU_TANH):
+        gelu = activation == engine.ACT_GELU_TANH
+        f = 0.5 * g * (1 + np.tanh(0.7978846 * (g + 0.044715 * g ** 3))) if gelu else g / (1 + np.exp(-g))
+        act = run_glu(eng, t, X, engine.DTYPE_BF16, engine.DTYPE_BF16, n_ff + 5, activation)
+        assert np.all(act[:, n_ff:] == 0)
+        # |f'| <= 1.13; half an ulp of bf16 on top, and the activation's own
+        # rounding (f32 tanh and exp: an absolute 2^-21 of g u)
+        slack = 1.13 * np.abs(u) * bg + np.abs(f) * bu + np.abs(g * u) * 2.0 ** -21
+        err = np.abs(act[:, :n_ff] - f * u)
+        assert np.all(err <= slack + (np.abs(f * u) + slack) * 2.0 ** -8 + 1e-38)
+    t.free()
+
+
 def test_gated_ffn_f32_x_and_bf16_act(eng):
     n_ff, cols = 300, 544
     gate, up, t = upload_gate_up(eng, "cb4", n_ff, cols, seed=3)

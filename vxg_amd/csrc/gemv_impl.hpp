@@ -352,8 +352,8 @@ __device__ __forceinline__ void read_x_lds(const uint16_t* s_xn, uint32_t k0, fl
   }
 }
 
-// Kernel: MT tokens (m >= M_rt are padding; more than one token runs on the
-// MFMA kernels of gemm_skinny_impl.hpp), RPW rows per wave, up to S steps per batch.  Gated epilogues take n_ff and the output
+// Kernel: MT tokens (1 or 2; m >= M_rt are padding), RPW rows per wave, up to
+// S steps per batch.  Gated epilogues take n_ff and the output
 // row stride; the plain epilogue ignores both.  NORM: the norm prologue above
 // (MT = 1, bf16 x staged in dynamic LDS of nsteps * kStep elements).
 // KS > 1 (split K): the workgroup's KS waves share its RPW rows, wave w
@@ -2013,11 +2013,14 @@ hipError_t launch_kind(const DevTensor& t, const void* x, bool x_bf16, uint32_t 
     if (t.rows >= 4096) return launch_r<KIND, 1, 2>(t, x, x_bf16, m, y, y_bf16, s);
     return launch_r<KIND, 1, 1>(t, x, x_bf16, m, y, y_bf16, s);
   }
+  if constexpr (KIND == KIND_G64)   // two_token_gemv (gemv.hip)
+    if (m == 2 && x_bf16) return launch_s<KIND, 2, 1, true>(t, x, m, y, y_bf16, s);
   return hipErrorInvalidValue;
 }
 
-// Gated gate/up GEMV of one token: one output (a gate row and its up row) per
-// wave, the generic kernel for every kind (more tokens: gemm_skinny.hip).
+// Gated gate/up GEMV of one token, and of two where two_token_glu (gemv.hip)
+// takes them: one output (a gate row and its up row) per wave, the generic
+// kernel for every kind (more tokens: gemm_skinny.hip).
 template <uint32_t KIND, int MT, int S, bool XBF16, int EPI>
 hipError_t launch_glu_t(const DevTensor& t, const void* x, uint32_t m, uint32_t n_ff, void* y, bool y_bf16,
                         uint32_t y_stride, hipStream_t s) {
@@ -2075,6 +2078,7 @@ hipError_t launch_glu_m(const DevTensor& t, const void* x, bool x_bf16, uint32_t
     if (m == 1 && try_glu_cb4_m1<EPI>(t, x, x_bf16, n_ff, y, y_bf16, y_stride, s, &e)) return e;
   }
   if (m == 1) return launch_glu_x<KIND, 1, EPI>(t, x, x_bf16, m, n_ff, y, y_bf16, y_stride, s);
+  if (m == 2 && x_bf16) return launch_glu_s<KIND, 2, true, EPI>(t, x, m, n_ff, y, y_bf16, y_stride, s);
   return hipErrorInvalidValue;
 }
 

@@ -37,6 +37,7 @@ hipError_t launch_gemv_norm(const DevTensor& t, const NormIn& nin, int epi, void
                             hipStream_t s);
 hipError_t launch_gemv_glu(const DevTensor& t, const void* x, bool x_bf16, uint32_t m, void* act, bool act_bf16,
                            uint32_t act_stride, bool gelu, hipStream_t s);
+bool two_token_glu(const DevTensor& t, uint32_t m, bool x_bf16, bool act_bf16);
 hipError_t launch_glu_act(const float* gu, uint32_t m, uint32_t n_ff, bool gelu, void* act, bool act_bf16,
                           uint32_t act_stride, hipStream_t s);
 hipError_t launch_rms_norm(float* cur, const float* delta, const float* w, void* out, bool out_bf16, uint32_t dim,
@@ -943,8 +944,8 @@ int vxt_hip_ffn_glu_dev(void* ctx, void* tensor, const void* x, uint32_t x_dtype
     hipStream_t s = static_cast<hipStream_t>(stream);
     const DevTensor d = t->dev();
     hipError_t e;
-    if (batch_m == 1) {
-      e = vxt::launch_gemv_glu(d, x, xb, 1, act, ab, act_stride, gelu, s);
+    if (batch_m == 1 || vxt::two_token_glu(d, batch_m, xb, ab)) {
+      e = vxt::launch_gemv_glu(d, x, xb, batch_m, act, ab, act_stride, gelu, s);
     } else {
       // The workspace of the staged form: the GEMM's own, then gate and up
       // rows in f32.  The fused forms use less of it or none; what a call
