@@ -57,6 +57,36 @@ def test_large_tile_edges(eng, kind, rows, cols, M, f32):
     t.free()
 
 
+@pytest.mark.parametrize("rows,cols,M", [(4000, 600, 129), (6144, 520, 1030), (2050, 4128, 192)])
+@pytest.mark.parametrize("kind", ["cb4", "g64", "q8", "q4_0"])
+def test_large_tile_f32_inf_rows(eng, kind, rows, cols, M):
+    """f32 activations with an Inf, or Infs of both signs, beside entries of
+    1e10, and a NaN: the reference's pattern of Inf and NaN outputs; the other
+    rows keep the file's bound."""
+    print(f"large tile f32 inf {kind} rows={rows} cols={cols} M={M}", flush=True)
+    m = synth.make_q40(rows, cols, seed=8) if kind == "q4_0" else make(kind, rows, cols, seed=8)
+    t = eng.upload_packed(m)
+    X = np.random.default_rng(M).standard_normal((M, cols)).astype(np.float32)
+    X[3] *= np.float32(1e10)
+    X[3, 17], X[M - 1, cols - 5], X[7, 0], X[7, cols - 1], X[9, cols // 2] = np.inf, -np.inf, np.inf, -np.inf, np.nan
+    eng.set_gemm_path(engine.GEMM_PANEL)
+    try:
+        got = run_dev(eng, t, X, engine.DTYPE_F32, M, engine.DTYPE_F32)
+    finally:
+        eng.set_gemm_path(engine.GEMM_AUTO)
+    t.free()
+    sel = [3, 7, 9, M - 1]
+    with np.errstate(all="ignore"):
+        pat = oracle.gemm(m, X[sel], threads=8)
+    y = got[sel]
+    assert np.array_equal(np.isnan(y), np.isnan(pat)) and np.array_equal(np.isinf(y), np.isinf(pat))
+    both = np.isinf(pat)
+    assert both.any() and np.array_equal(np.sign(y[both]), np.sign(pat[both]))
+    fin = np.setdiff1d(np.arange(M), sel)
+    Xf, W = X[fin].astype(np.float64), oracle.decode_rows(m).astype(np.float64)
+    assert np.all(np.abs(got[fin] - Xf @ W.T) <= bound_of(Xf, W, cols))
+
+
 # Gated [gate; up] calls in one K range: batch and outputs that end inside a
 # tile, output counts that are and are not multiples of 8 pieces, 4- and 8-wave
 # workgroups and 256 x 192 tiles.  Bound: an output is act(g) u with g and u

@@ -208,3 +208,112 @@ def test_g64_all_of_k_in_one_range(eng, rows, cols, M):
     t.free()
     W = oracle.decode_rows(m).astype(np.float64)
     assert np.all(np.abs(got - X @ W.T) <= (160 + cols / 128) * 2.0 ** -24 * (np.abs(X) @ np.abs(W).T))
+
+
+FORMS = [(70, 544, 5, False), (70, 4160, 7, False), (4200, 300, 5, False), (40, 2600, 16, False), (40, 2600, 40, False),
+         (70, 2100, 5, True), (4200, 700, 3, True), (70, 2600, 12, True), (32800, 288, 12, False)]
+
+
+@pytest.mark.parametrize("kind", ["cb4", "g64", "q8", "q4_0"])
+@pytest.mark.parametrize("rows,cols,M,f32", FORMS + [(67, 2047, 2, False), (33, 1031, 33, False)])
+def test_skinny_single_products(eng, kind, rows, cols, M, f32):
+    """One activation per token is not zero, at the first and last column and
+    over the chunks between: an output is one product, of operands with all
+    24 bits set where they have them (cb4's centroids, f32 activations), and may
+    not miss the lowest of their three terms.  At most four roundings (the
+    term sums, a scale, the result); products of the terms left out are below
+    2^-24 of it, twice."""
+    print(f"skinny single {kind} rows={rows} cols={cols} M={M} f32={f32}", flush=True)
+    m = synth.make_q40(rows, cols, seed=3) if kind == "q4_0" else make(kind, rows, cols, seed=3)
+    if kind == "cb4":
+        m.centroids[:] = (m.centroids.view(np.uint32) | 0xFF).view(np.float32)
+    t = eng.upload_packed(m)
+    X = np.zeros((M, cols), np.float32)
+    at = np.linspace(0, cols - 1, M).astype(int)
+    x = 1 + np.random.default_rng(cols).random(M).astype(np.float32)
+    X[np.arange(M), at] = (x.view(np.uint32) | 0xFF).view(np.float32) if f32 else bf16_bits_to_f32(f32_to_bf16_bits(x))
+    got = run_dev(eng, t, X if f32 else f32_to_bf16_bits(X), engine.DTYPE_F32 if f32 else engine.DTYPE_BF16, M,
+                  engine.DTYPE_F32)
+    t.free()
+    W = oracle.decode_rows(m)[:, at].astype(np.float64).T
+    xs = X[np.arange(M), at].astype(np.float64)[:, None]
+    # a residual is a product of its own: its column's weight is a sum
+    mag = np.abs(W * xs)
+    if kind == "cb4":
+        mag = mag + 0.1 * np.abs(xs) * np.isin(at, m.outliers_packed & 0xFFFF)[:, None]
+    bound = 6 * 2.0 ** -24 * mag
+    assert np.all(np.abs(got - W * xs) <= bound)
+    # ... and the bound shows a lost third term
+    if kind == "cb4" or f32:
+        lost = (X.view(np.uint32) & 0xFFFFFF00).view(np.float32)[np.arange(M), at].astype(np.float64)[:, None] if f32 else \
+            xs * (1 - 2.0 ** -17)
+        assert np.any(np.abs(W * lost - W * xs) > bound)
+
+
+def _nibbles(b):
+    return np.stack([b & 15, b >> 4], -1).reshape(-1)
+
+
+def _nonfinite(m, kind):
+    """Inf and NaN in tables and scales of a few rows; returns the rows that
+    have any.  Padded columns keep finite entries; cb4's shared table has its Inf
+    at entry 0, which no other row's columns hold."""
+    rows, cols = m.rows, m.cols
+    if kind == "cb4":
+        q = _nibbles(m.packed_words.view(np.uint8)).reshape(rows, -1)
+        q[q == 0], q[q == 7] = 1, 8
+        q[2, 5], q[3, cols - 1], q[6, cols // 2] = 0, 0, 7
+        b = q.reshape(-1, 2)
+        m.packed_words[:] = np.ascontiguousarray(b[:, 0] | b[:, 1] << 4).astype(np.uint8).view(np.uint32)
+        m.centroids[0], m.centroids[7] = np.inf, np.nan
+        s = m.scales_f16.reshape(rows, -1)
+        s[9, 0], s[11, (cols - 1) // 128] = 0x7C00, 0x7E00
+        return [2, 3, 6, 9, 11]
+    if kind == "g64":
+        q = _nibbles(m.idx).reshape(rows, -1)
+        last = (cols - 1) // 64
+        q[q == 3], q[:, cols:] = 4, 1
+        q[2, 5], q[3, cols - 1], q[6, cols - 1] = 3, 3, 3
+        b = q.reshape(-1, 2)
+        m.idx[:] = (b[:, 0] | b[:, 1] << 4).reshape(m.idx.shape)
+        L = m.lut_f16.reshape(rows, -1, 16)
+        L[2, 0, 3], L[3, last, 3], L[6, last, 3], L[9, last, 3] = 0x7C00, 0xFC00, 0x7E00, 0x7C00
+        return [2, 3, 6]
+    if kind == "q8":
+        s = m.blocks.reshape(rows, -1, 34)[:, :, :2].copy().view(np.uint16)[:, :, 0]
+    else:
+        s = m.scales_f16.reshape(rows, -1)
+    s[2, 0], s[3, (cols - 1) // 32], s[6, (cols - 1) // 64] = 0x7C00, 0xFC00, 0x7E00
+    if kind == "q8":
+        m.blocks.reshape(rows, -1, 34)[:, :, :2] = np.ascontiguousarray(s)[:, :, None].view(np.uint8)
+        m.blocks.reshape(rows, -1, 34)[2, 0, 2:] = 5
+    else:
+        m.qs_words.reshape(rows, -1, 4)[2, 0] = 0x9B9B9B9B
+    return [2, 3, 6]
+
+
+@pytest.mark.parametrize("kind", ["cb4", "g64", "q8", "q4_0"])
+@pytest.mark.parametrize("rows,cols,M,f32", FORMS)
+def test_skinny_nonfinite_tables_and_scales(eng, kind, rows, cols, M, f32):
+    """Inf and NaN in codebooks, centroids and scales reach the outputs that
+    the reference's loops give them to, and no others."""
+    print(f"skinny nonfinite weights {kind} rows={rows} cols={cols} M={M} f32={f32}", flush=True)
+    m = synth.make_q40(rows, cols, seed=12) if kind == "q4_0" else make(kind, rows, cols, seed=12)
+    bad = _nonfinite(m, kind)
+    t = eng.upload_packed(m)
+    X = np.random.default_rng(M).standard_normal((M, cols)).astype(np.float32)
+    X[0], X[1, ::3] = np.abs(X[0]) + 0.5, 0
+    xh = X if f32 else f32_to_bf16_bits(X)
+    Xq = X if f32 else bf16_bits_to_f32(xh).reshape(M, cols)
+    got = run_dev(eng, t, xh, engine.DTYPE_F32 if f32 else engine.DTYPE_BF16, M, engine.DTYPE_F32)
+    t.free()
+    with np.errstate(all="ignore"):
+        pat = oracle.gemm(m, Xq, threads=8) if M > 8 else np.stack([oracle.gemv(m, x, threads=8) for x in Xq])
+        W = oracle.decode_rows(m).astype(np.float64)
+    assert not np.isfinite(pat[0, bad]).any() and np.isinf(pat[0, bad]).any()
+    assert np.array_equal(np.isnan(got), np.isnan(pat)) and np.array_equal(np.isinf(got), np.isinf(pat))
+    both = np.isinf(pat)
+    assert np.array_equal(np.sign(got[both]), np.sign(pat[both]))
+    good = np.setdiff1d(np.arange(rows), bad)
+    W, Xf = W[good], Xq.astype(np.float64)
+    assert np.all(np.abs(got[:, good] - Xf @ W.T) <= (160 + cols / 128) * 2.0 ** -24 * (np.abs(Xf) @ np.abs(W).T))
