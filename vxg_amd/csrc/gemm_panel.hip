@@ -906,11 +906,13 @@ inline Plan plan(const DevTensor& t, uint32_t m, bool x_bf16, bool lib) {
   // 55.7 / 67.9 (96.0 / 76.8 / 92.8).  Up to 128 tokens, and below 32 tiles (64 up to
   // 191 tokens), the other's 64-row tiles fill more of the chip; up to 255 tokens
   // also with K < 1024 (191 tokens 512 -> 6144 30.6 / 21.3 / 28.9 against 26.3 / 17.6 /
-  // 24.8; g64 up to 128 tiles of K = 1024: 1024 -> 4096 27.5 against 23.5), up to 191 where two MFMAs more per product make the empty rows of 128-row
-  // tiles dear (hi/lo panels of 128 M weights: 130 tokens 8192 -> 16384 cb4 526 against
-  // 472, Q8 444 against 402, Q4_0 466 against 419; g64 233 against 296).
+  // 24.8; g64 up to 128 tiles of K = 1024: 1024 -> 4096 27.5 against 23.5), up to 191
+  // where two MFMAs more per product make the empty rows of 128-row tiles dear (hi/lo
+  // panels of 128 M weights: 130 tokens 8192 -> 16384 cb4 526 against 472, Q8 444
+  // against 402, Q4_0 466 against 419; g64 233 against 296).
   const size_t weights = (size_t)t.cols * t.rows;
-  const bool deep = m >= 256 || (t.cols >= 1024 && !(t.kind == KIND_G64 && t.cols == 1024 && t128 <= 128) && !(m < 192 && pl.wmode != kWPlain && weights >= (size_t)128000000));
+  const bool deep = m >= 256 || (t.cols >= 1024 && !(t.kind == KIND_G64 && t.cols == 1024 && t128 <= 128) &&
+                                 !(m < 192 && pl.wmode != kWPlain && weights >= (size_t)128000000));
   if (!x_bf16 && !lib && m > 128 && t128 >= (m >= 192 ? 32u : 64u) && deep && fits) {
     pl.d3mode = pl.wmode == kWPlain ? 0 : 1;
     pl.d3cfg = ((m + 255) / 256) * ((t.rows + 127) / 128) * pl.splits >= 192 ? 4 : 3;

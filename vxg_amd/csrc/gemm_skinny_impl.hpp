@@ -1053,8 +1053,10 @@ hipError_t launch_glu(const DevTensor& t, const Args& a, bool x_bf16, hipStream_
     return M <= 4 ? launch<KIND, 3, 1, 4, 1, N1, true, true>(t, a, n, s)
                   : launch<KIND, 3, 1, 16, G ? 2 : 1, 1, true, true>(t, a, n, s);
   }
-  // Half tiles for the sizes where the plain form takes them: the sums are
-  // those of the plain form, bit for bit (up to 8 tokens).
+  // Half tiles for the sizes where the plain form takes them: up to 8 tokens the
+  // sums are those of the plain form's skinny_kernel, bit for bit (not those of
+  // its streaming form from kStreamRows, nor of the kernels that launch_gemv
+  // keeps for two tokens of g64 and of Q8_0).
   if (M <= 8 && t.rows <= kHalfRows && (!G || K > 2048)) {
     if constexpr (!G)
       if (K <= 2048)

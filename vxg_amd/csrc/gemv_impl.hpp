@@ -659,31 +659,21 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t x_row_rsrc(const uint16_t* x, 
                                            (int)(cols * 2u), 0x00020000);
 }
 
-__device__ __forceinline__ void load_x_pairs(__amdgpu_buffer_rsrc_t r, uint32_t k0, uint32_t x_vec,
-                                             uint32_t (&xp)[kChunk / 2]) {
-  if (x_vec) {   // cols % 8 == 0: each 16-byte piece is wholly inside or outside the row
+__device__ __forceinline__ void load_x_pairs(__amdgpu_buffer_rsrc_t r, uint32_t k0, uint32_t (&xp)[kChunk / 2]) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, (k0 + 8u * i) * 2u, 0, 0);
-      xp[4 * i + 0] = v.x;
-      xp[4 * i + 1] = v.y;
-      xp[4 * i + 2] = v.z;
-      xp[4 * i + 3] = v.w;
-    }
-  } else {
-#pragma unroll
-    for (int j = 0; j < kChunk / 2; ++j) {
-      const uint32_t v0 = __builtin_amdgcn_raw_buffer_load_b16(r, (k0 + 2u * j) * 2u, 0, 0);
-      const uint32_t v1 = __builtin_amdgcn_raw_buffer_load_b16(r, (k0 + 2u * j + 1u) * 2u, 0, 0);
-      xp[j] = (v0 & 0xffffu) | (v1 << 16);
-    }
+  for (int i = 0; i < 4; ++i) {   // cols % 8 == 0: each 16-byte piece is wholly inside or outside the row
+    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, (k0 + 8u * i) * 2u, 0, 0);
+    xp[4 * i + 0] = v.x;
+    xp[4 * i + 1] = v.y;
+    xp[4 * i + 2] = v.z;
+    xp[4 * i + 3] = v.w;
   }
 }
 
 template <int MT, int RPW, int S>
 __global__ __launch_bounds__(kWaves * 64) void gemv_q8_dot2_kernel(DevTensor t, const uint16_t* __restrict__ x,
                                                                   void* __restrict__ y, uint32_t M_rt,
-                                                                  uint32_t y_bf16, uint32_t x_vec) {
+                                                                  uint32_t y_bf16) {
   const uint32_t lane = threadIdx.x & 63;
   const uint32_t wave = threadIdx.x >> 6;
   const uint32_t row0 = (blockIdx.x * kWaves + wave) * RPW;
@@ -708,7 +698,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemv_q8_dot2_kernel(DevTensor t, 
       if ((uint32_t)s < ns) {
         const uint32_t k0 = (s0 + s) * kStep + lane * kChunk;
 #pragma unroll
-        for (int m = 0; m < MT; ++m) load_x_pairs(x_row_rsrc(x, cols, (uint32_t)m < M_rt ? m : 0), k0, x_vec, xp[s][m]);
+        for (int m = 0; m < MT; ++m) load_x_pairs(x_row_rsrc(x, cols, (uint32_t)m < M_rt ? m : 0), k0, xp[s][m]);
         const uint32_t k0c = k0 < kp ? k0 : kp - kChunk;
 #pragma unroll
         for (int r = 0; r < RPW; ++r) {
@@ -751,117 +741,6 @@ __global__ __launch_bounds__(kWaves * 64) void gemv_q8_dot2_kernel(DevTensor t, 
           static_cast<uint16_t*>(y)[(size_t)m * rows + row] = f32_to_bf16(v);
         else
           static_cast<float*>(y)[(size_t)m * rows + row] = v;
-      }
-    }
-  }
-}
-
-// Larger batches (M >= 4): the same dot2 arithmetic with the activations
-// staged in LDS once per workgroup.  Reading x straight from L2 costs
-// M * K * 2 bytes per wave, which at M = 8 is four times the weight bytes a
-// wave streams, and L2 bandwidth, not HBM, sets the time.  Workgroups are
-// persistent: each stages x (all M tokens, all of K: kp <= 3 * kStep) once and
-// then walks row blocks with a stride of the grid size.
-template <int MT, int RPW, int WAVES, int NS>
-__global__ __launch_bounds__(WAVES * 64) void gemv_q8_lds_kernel(DevTensor t, const uint16_t* __restrict__ x,
-                                                                void* __restrict__ y, uint32_t M_rt,
-                                                                uint32_t y_bf16, uint32_t x_vec) {
-  extern __shared__ __attribute__((aligned(16))) uint32_t s_x[];   // [MT][kp / 2] packed bf16 pairs
-  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const uint32_t rows = t.rows, cols = t.cols, kp = t.kp;
-  const uint32_t kpw = kp / 2;
-  const uint32_t nblocks = (rows + WAVES * RPW - 1) / (WAVES * RPW);
-
-  // First row block's weights go out before the activations are staged.
-  WChunk<KIND_Q8> wc[NS][RPW];
-  auto issue = [&](uint32_t b) {
-#pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      const uint32_t k0 = s * kStep + lane * kChunk;
-      const uint32_t k0c = k0 < kp ? k0 : kp - kChunk;
-#pragma unroll
-      for (int r = 0; r < RPW; ++r) {
-        const uint32_t row = (b * WAVES + wave) * RPW + r;
-        load_chunk<KIND_Q8>(t, row < rows ? row : rows - 1, k0c, 0, 0, wc[s][r]);
-      }
-    }
-  };
-  if (blockIdx.x < nblocks) issue(blockIdx.x);
-
-  // Stage x: 8-column pieces, zero outside [0, cols) (raw-buffer bounds).
-  const uint32_t ppr = kp / 8;   // pieces per token row
-  for (uint32_t p = tid; p < MT * ppr; p += WAVES * 64) {
-    const uint32_t m = p / ppr, pc = p - m * ppr;
-    const __amdgpu_buffer_rsrc_t r = x_row_rsrc(x, cols, m < M_rt ? m : 0);
-    u32x4 v;
-    if (x_vec) {
-      v = __builtin_amdgcn_raw_buffer_load_b128(r, pc * 16u, 0, 0);
-    } else {
-      uint32_t h[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) h[j] = __builtin_amdgcn_raw_buffer_load_b16(r, (pc * 8u + j) * 2u, 0, 0) & 0xffffu;
-      v = u32x4{h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16)};
-    }
-    *reinterpret_cast<u32x4*>(&s_x[m * kpw + pc * 4]) = v;
-  }
-  __syncthreads();
-
-  for (uint32_t b = blockIdx.x; b < nblocks; b += gridDim.x) {
-    float acc[RPW][MT];
-#pragma unroll
-    for (int r = 0; r < RPW; ++r)
-#pragma unroll
-      for (int m = 0; m < MT; ++m) acc[r][m] = 0.0f;
-#pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      const uint32_t k0 = s * kStep + lane * kChunk;
-      const bool kin = k0 < kp;
-      const uint32_t k0c = kin ? k0 : kp - kChunk;
-      uint32_t qp[RPW][kChunk / 2];
-      float d[RPW];
-#pragma unroll
-      for (int r = 0; r < RPW; ++r) {
-        q8_pairs(wc[s][r], qp[r]);
-        d[r] = f16_to_f32(wc[s][r].d);
-      }
-#pragma unroll
-      for (int m = 0; m < MT; ++m) {
-        uint32_t xp[kChunk / 2];
-        const u32x4* src = reinterpret_cast<const u32x4*>(&s_x[m * kpw + k0c / 2]);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const u32x4 v = src[i];
-          xp[4 * i] = v.x;
-          xp[4 * i + 1] = v.y;
-          xp[4 * i + 2] = v.z;
-          xp[4 * i + 3] = v.w;
-        }
-#pragma unroll
-        for (int r = 0; r < RPW; ++r) {
-          float p0 = 0.0f, p1 = 0.0f;
-#pragma unroll
-          for (int j = 0; j < kChunk / 2; j += 2) {
-            p0 = dot2_bf16(qp[r][j], xp[j], p0);
-            p1 = dot2_bf16(qp[r][j + 1], xp[j + 1], p1);
-          }
-          acc[r][m] += kin ? (p0 + p1) * d[r] : 0.0f;
-        }
-      }
-    }
-    const uint32_t row0 = (b * WAVES + wave) * RPW;
-    if (b + gridDim.x < nblocks) issue(b + gridDim.x);   // next block's weights in flight during the reduction
-#pragma unroll
-    for (int r = 0; r < RPW; ++r) {
-      const uint32_t row = row0 + r;
-#pragma unroll
-      for (int m = 0; m < MT; ++m) {
-        const float v = wave_sum(acc[r][m]);
-        if (lane == 0 && row < rows && (uint32_t)m < M_rt) {
-          if (y_bf16)
-            static_cast<uint16_t*>(y)[(size_t)m * rows + row] = f32_to_bf16(v);
-          else
-            static_cast<float*>(y)[(size_t)m * rows + row] = v;
-        }
       }
     }
   }
@@ -1720,58 +1599,14 @@ hipError_t launch_q8_lm(const DevTensor& t, const void* x, uint32_t m, void* y, 
 constexpr uint32_t kQ8M8MaxNb = 256;
 hipError_t launch_q8_m8(const DevTensor& t, const void* x, uint32_t m, void* y, bool y_bf16, hipStream_t s);
 
-// Grid for the persistent kernel: enough workgroups to fill every CU at the
-// occupancy the LDS footprint allows, never more than there are row blocks.
-template <int MT, int RPW, int WAVES, int NS>
-hipError_t launch_q8_lds_t(const DevTensor& t, const void* x, uint32_t m, void* y, bool y_bf16, hipStream_t s,
-                           uint32_t per_cu = 0) {
-  // Dynamic LDS above 64 KiB must be allowed per kernel, once.
-  static const hipError_t attr = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(&gemv_q8_lds_kernel<MT, RPW, WAVES, NS>),
-      hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-  if (attr != hipSuccess) return attr;
-  const size_t lds = (size_t)MT * t.kp * 2;
-  if (lds > 160u * 1024u || (t.kp + kStep - 1) / kStep != (uint32_t)NS) return hipErrorInvalidValue;
-  const uint32_t nblocks = (t.rows + WAVES * RPW - 1) / (WAVES * RPW);
-  uint32_t occ = per_cu ? per_cu : (uint32_t)std::min<size_t>(160u * 1024u / lds, 16u / WAVES * 2u);
-  if (occ == 0) occ = 1;
-  const uint32_t grid = std::min<uint32_t>(nblocks, 256u * occ);
-  const uint32_t x_vec = (reinterpret_cast<uintptr_t>(x) % 16 == 0) && t.cols % 8 == 0;
-  hipLaunchKernelGGL((gemv_q8_lds_kernel<MT, RPW, WAVES, NS>), dim3(grid), dim3(WAVES * 64), lds, s, t,
-                     static_cast<const uint16_t*>(x), y, m, (uint32_t)(y_bf16 ? 1u : 0u), x_vec);
-  return hipGetLastError();
-}
-
 template <int MT, int RPW, int S>
 hipError_t launch_q8_dot2_t(const DevTensor& t, const void* x, uint32_t m, void* y, bool y_bf16, hipStream_t s) {
+  if (reinterpret_cast<uintptr_t>(x) % 16 != 0 || t.cols % 8 != 0) return hipErrorInvalidValue;
   const uint32_t rows_per_block = kWaves * RPW;
   const dim3 grid((t.rows + rows_per_block - 1) / rows_per_block);
-  const uint32_t x_vec = (reinterpret_cast<uintptr_t>(x) % 16 == 0) && t.cols % 8 == 0;
   hipLaunchKernelGGL((gemv_q8_dot2_kernel<MT, RPW, S>), grid, dim3(kWaves * 64), 0, s, t,
-                     static_cast<const uint16_t*>(x), y, m, (uint32_t)(y_bf16 ? 1u : 0u), x_vec);
+                     static_cast<const uint16_t*>(x), y, m, (uint32_t)(y_bf16 ? 1u : 0u));
   return hipGetLastError();
-}
-
-// Shape choices for Q8 x bf16 at M = 2..8, from measurements over the
-// decode shapes (K x N in {2048, 6144} x {2048, 6144}, and the 151936-row LM
-// head): the LDS-staged persistent kernel wins only when there are many more
-// row blocks than CUs; otherwise the direct kernel with two rows per wave.
-template <int MT>
-hipError_t launch_q8_dot2_m(const DevTensor& t, const void* x, uint32_t m, void* y, bool y_bf16, hipStream_t s) {
-  const uint32_t nsteps = (t.kp + kStep - 1) / kStep;
-  if (t.rows >= 65536 && nsteps == 1) {
-    if constexpr (MT >= 8) return launch_q8_lds_t<MT, 1, 4, 1>(t, x, m, y, y_bf16, s);
-    return launch_q8_lds_t<MT, 2, 8, 1>(t, x, m, y, y_bf16, s);
-  }
-  if constexpr (MT == 2) {
-    if (nsteps == 3) return launch_q8_dot2_t<2, 1, 1>(t, x, m, y, y_bf16, s);
-    if (nsteps >= 2) return launch_q8_dot2_t<2, 2, 2>(t, x, m, y, y_bf16, s);
-    return launch_q8_dot2_t<2, 2, 1>(t, x, m, y, y_bf16, s);
-  } else if constexpr (MT == 4) {
-    if (nsteps >= 2) return launch_q8_dot2_t<4, 2, 2>(t, x, m, y, y_bf16, s);
-    return launch_q8_dot2_t<4, 2, 1>(t, x, m, y, y_bf16, s);
-  }
-  return launch_q8_dot2_t<MT, 2, 1>(t, x, m, y, y_bf16, s);
 }
 
 template <uint32_t KIND, int MT, int RPW, int S, bool XBF16>
@@ -1934,7 +1769,7 @@ hipError_t launch_kind(const DevTensor& t, const void* x, bool x_bf16, uint32_t 
       }
     }
     if (x_bf16 && m >= 2) {
-      if (m == 2) return launch_q8_dot2_m<2>(t, x, m, y, y_bf16, s);
+      if (m == 2) return launch_q8_dot2_t<2, 2, 2>(t, x, m, y, y_bf16, s);
       if (m > 4 && t.cols % 8 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && t.kp / 32 <= kQ8MfmaMaxNb<4, 4>)
         return launch_q8_mfma_t<4, 4>(t, x, m, y, y_bf16, s);
       // Rows longer than two K steps at 5..8 tokens: the 8-row MFMA kernel,
@@ -1946,8 +1781,8 @@ hipError_t launch_kind(const DevTensor& t, const void* x, bool x_bf16, uint32_t 
       if (m > 4 && t.cols % 8 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && t.kp > 2 * kStep &&
           t.kp / 32 <= kQ8M8MaxNb && t.rows <= 4096)
         return launch_q8_m8(t, x, m, y, y_bf16, s);
-      if (m <= 4) return launch_q8_dot2_m<4>(t, x, m, y, y_bf16, s);
-      if (m <= 8) return launch_q8_dot2_m<8>(t, x, m, y, y_bf16, s);
+      if (m <= 4) return launch_q8_dot2_t<4, 2, 2>(t, x, m, y, y_bf16, s);
+      if (m <= 8) return launch_q8_dot2_t<8, 2, 1>(t, x, m, y, y_bf16, s);
       return hipErrorInvalidValue;
     }
   }
@@ -2013,8 +1848,8 @@ hipError_t launch_kind(const DevTensor& t, const void* x, bool x_bf16, uint32_t 
     if (t.rows >= 4096) return launch_r<KIND, 1, 2>(t, x, x_bf16, m, y, y_bf16, s);
     return launch_r<KIND, 1, 1>(t, x, x_bf16, m, y, y_bf16, s);
   }
-  if constexpr (KIND == KIND_G64)   // two_token_gemv (gemv.hip)
-    if (m == 2 && x_bf16) return launch_s<KIND, 2, 1, true>(t, x, m, y, y_bf16, s);
+  if constexpr (KIND == KIND_G64)   // two_token_gemv (gemv.hip): K <= 2048, one step
+    if (m == 2 && x_bf16 && t.kp <= kStep) return launch_t<KIND, 2, 1, 1, true>(t, x, m, y, y_bf16, s);
   return hipErrorInvalidValue;
 }
 
