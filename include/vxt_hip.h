@@ -560,12 +560,13 @@ VXT_API int vxt_hip_last_kernel_ms(void* ctx, double* ms);
  * measured speed: every kind takes the few-token MFMA kernels up to batch_m
  * 16 (unless their partial sums need more than the workspace of the other
  * paths: g64 and Q8_0 of many rows and cols > 2048), and to 32 or 64 by kind
- * and size; above, g64 weights with bf16
+ * and size, whatever workspace the context holds; above, g64 weights with bf16
  * activations decode inside the MFMA loop -- the fused kernel up to batch_m 64,
- * the 128 x 128 tile kernel above, to 767 (1023 when cols > rows); cb4 weights with bf16
- * activations take the cb4 tile kernel described under FUSED from batch_m 128
- * to 511 when the tensor is eligible for it; Q8_0 (and Q4_0) weights with
- * bf16 activations and batch_m <= 128 take the fused kernel; every other call
+ * the 128 x 128 tile kernel above, to 767 (1023 when cols > rows); cb4 weights
+ * with bf16 activations take the cb4 tile kernel described under FUSED from
+ * batch_m 128 to 511 (255 when cols < rows) when the tensor is eligible for it;
+ * Q8_0 weights with bf16 activations take the fused kernel to batch_m 128 (511
+ * when cols >= rows); every other call
  * takes the two-phase path (a decoded f16 weight panel, then the dense MFMA
  * kernel).  PANEL pins the two-phase path.  FUSED takes the decode-in-loop
  * kernels wherever they apply: for cb4 weights with bf16 activations the cb4
@@ -573,7 +574,7 @@ VXT_API int vxt_hip_last_kernel_ms(void* ctx, double* ms);
  * the MFMA loop, no weight panel), when the upload found the tensor eligible
  * (every plane finite, each row's residual columns strictly increasing, at
  * most 16384 residuals per block of 128 rows); for g64 the tile kernel above
- * batch_m 64 and the fused kernel below; for Q8_0 / Q4_0 the fused kernel;
+ * batch_m 64 and the fused kernel below; for Q8_0 the fused kernel;
  * the two-phase path otherwise.  LIBRARY pins the two-phase path with its
  * dense phase on hipBLASLt, a comparison only (falling back to the own
  * kernel for a shape the library has no algorithm for).  A tuning and test
