@@ -901,7 +901,7 @@ inline Plan plan(const DevTensor& t, uint32_t m, bool x_bf16, bool lib) {
   // workgroup per CU while a range keeps 8 K tiles; 256 x 128 tiles of 8 waves
   // where these and their ranges fill the chip, else 128 x 128.  Whole call, us,
   // cb4 / g64 / Q8, against the register-staged kernel: 500 tokens 2048 -> 2048
-  // 35.6 / 30.2 / 33.8 (41.0 / 33.3 / 39.0); 300, 2048 -> 6144 60.4 / 42.8 / 55.6
+  // 35.6 / 30.2 / 35.0 (41.0 / 33.3 / 39.0); 300, 2048 -> 6144 60.4 / 42.8 / 55.6
   // (90.3 / 67.5 / 86.8; 64.5 / 44.5 / 60.1 on 128 x 128); 2048, 2048 -> 2048 71.3 /
   // 55.7 / 67.9 (96.0 / 76.8 / 92.8).  Up to 128 tokens, and below 32 tiles (64 up to
   // 191 tokens), the other's 64-row tiles fill more of the chip; up to 255 tokens
