@@ -654,26 +654,40 @@ __device__ __forceinline__ void q8_pairs(const WChunk<KIND_Q8>& c, uint32_t (&qp
 // [0, cols).  The token's row is a raw buffer (base and byte size in SGPRs):
 // offsets are 32-bit per lane, and the hardware returns zeros for any part
 // of a load at or past the row's end, so no clamping or masking is needed.
+// launch_gemv sends only 16-byte rows here; the two-byte loads stay because the
+// branch holds the tokens' loads in front of the weights': without it the
+// compiler moves them to their uses (8 tokens 12288 -> 40000 282 -> 363 us, still
+// 288 and 6144 rows 8 % slower with scheduling barriers in its place).
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t x_row_rsrc(const uint16_t* x, uint32_t cols, uint32_t m) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(x + (size_t)m * cols), (short)0,
                                            (int)(cols * 2u), 0x00020000);
 }
 
-__device__ __forceinline__ void load_x_pairs(__amdgpu_buffer_rsrc_t r, uint32_t k0, uint32_t (&xp)[kChunk / 2]) {
+__device__ __forceinline__ void load_x_pairs(__amdgpu_buffer_rsrc_t r, uint32_t k0, uint32_t x_vec,
+                                             uint32_t (&xp)[kChunk / 2]) {
+  if (x_vec) {   // cols % 8 == 0: each 16-byte piece is wholly inside or outside the row
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {   // cols % 8 == 0: each 16-byte piece is wholly inside or outside the row
-    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, (k0 + 8u * i) * 2u, 0, 0);
-    xp[4 * i + 0] = v.x;
-    xp[4 * i + 1] = v.y;
-    xp[4 * i + 2] = v.z;
-    xp[4 * i + 3] = v.w;
+    for (int i = 0; i < 4; ++i) {
+      const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, (k0 + 8u * i) * 2u, 0, 0);
+      xp[4 * i + 0] = v.x;
+      xp[4 * i + 1] = v.y;
+      xp[4 * i + 2] = v.z;
+      xp[4 * i + 3] = v.w;
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < kChunk / 2; ++j) {
+      const uint32_t v0 = __builtin_amdgcn_raw_buffer_load_b16(r, (k0 + 2u * j) * 2u, 0, 0);
+      const uint32_t v1 = __builtin_amdgcn_raw_buffer_load_b16(r, (k0 + 2u * j + 1u) * 2u, 0, 0);
+      xp[j] = (v0 & 0xffffu) | (v1 << 16);
+    }
   }
 }
 
 template <int MT, int RPW, int S>
 __global__ __launch_bounds__(kWaves * 64) void gemv_q8_dot2_kernel(DevTensor t, const uint16_t* __restrict__ x,
                                                                   void* __restrict__ y, uint32_t M_rt,
-                                                                  uint32_t y_bf16) {
+                                                                  uint32_t y_bf16, uint32_t x_vec) {
   const uint32_t lane = threadIdx.x & 63;
   const uint32_t wave = threadIdx.x >> 6;
   const uint32_t row0 = (blockIdx.x * kWaves + wave) * RPW;
@@ -698,7 +712,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemv_q8_dot2_kernel(DevTensor t, 
       if ((uint32_t)s < ns) {
         const uint32_t k0 = (s0 + s) * kStep + lane * kChunk;
 #pragma unroll
-        for (int m = 0; m < MT; ++m) load_x_pairs(x_row_rsrc(x, cols, (uint32_t)m < M_rt ? m : 0), k0, xp[s][m]);
+        for (int m = 0; m < MT; ++m) load_x_pairs(x_row_rsrc(x, cols, (uint32_t)m < M_rt ? m : 0), k0, x_vec, xp[s][m]);
         const uint32_t k0c = k0 < kp ? k0 : kp - kChunk;
 #pragma unroll
         for (int r = 0; r < RPW; ++r) {
@@ -1601,11 +1615,11 @@ hipError_t launch_q8_m8(const DevTensor& t, const void* x, uint32_t m, void* y, 
 
 template <int MT, int RPW, int S>
 hipError_t launch_q8_dot2_t(const DevTensor& t, const void* x, uint32_t m, void* y, bool y_bf16, hipStream_t s) {
-  if (reinterpret_cast<uintptr_t>(x) % 16 != 0 || t.cols % 8 != 0) return hipErrorInvalidValue;
   const uint32_t rows_per_block = kWaves * RPW;
   const dim3 grid((t.rows + rows_per_block - 1) / rows_per_block);
+  const uint32_t x_vec = (reinterpret_cast<uintptr_t>(x) % 16 == 0) && t.cols % 8 == 0;
   hipLaunchKernelGGL((gemv_q8_dot2_kernel<MT, RPW, S>), grid, dim3(kWaves * 64), 0, s, t,
-                     static_cast<const uint16_t*>(x), y, m, (uint32_t)(y_bf16 ? 1u : 0u));
+                     static_cast<const uint16_t*>(x), y, m, (uint32_t)(y_bf16 ? 1u : 0u), x_vec);
   return hipGetLastError();
 }
 
